@@ -191,3 +191,38 @@ def test_abi_pool_softmax_bmm():
         ref = np.empty(bb * m * n, np.uint16)
         L.ivo_bmm(a[b * bb * m * k:(b + 1) * bb * m * k], bm[b * bb * k * n:(b + 1) * bb * k * n], ref, bb, m, k, n)
         assert _ok(got[b], ref, "bmm")
+
+
+@pytest.mark.parametrize("k,c,h,w,batch,off", [
+    (5, 128, 20, 20, 3, 0),    # five planes a work-group, the last group partial
+    (5, 3, 1, 1, 1, 0),        # the smallest plane
+    (5, 7, 13, 17, 2, 0),      # odd width: single-element loads and stores
+    (5, 6, 9, 10, 2, 1),       # even width at an odd element offset
+    (3, 5, 4, 6, 2, 0),        # three-wide windows, one register block of rows
+    (3, 2, 5, 3, 1, 0),
+    (5, 2, 200, 160, 1, 0),    # three bands of rows per plane
+    (5, 1, 9, 4001, 1, 0),     # rows so wide that a band is one register block
+    (3, 1, 6, 9000, 1, 0),     # wider than a band: the scalar kernel
+])
+def test_abi_maxpool_planes(k, c, h, w, batch, off):
+    """Stride-1 same-size max pools on planes, with infinities and NaNs among the values:
+    bit for bit the fmaxf chain from below every fp16 value (NaN taps ignored)."""
+    rng = np.random.default_rng(k * 1000 + w)
+    x = rng.standard_normal((batch, c, h, w)).astype(np.float16)
+    for v in (np.inf, -np.inf, np.nan):
+        x[rng.random(x.shape) < 0.02] = v
+    x.reshape(-1)[: min(x.size, 40)] = np.nan  # a window of nothing but NaN
+    p = k // 2
+    z = np.pad(np.where(np.isnan(x), np.float16(-np.inf), x), ((0, 0), (0, 0), (p, p), (p, p)),
+               constant_values=-np.inf)
+    ref = np.full_like(x, -np.inf)
+    for i in range(k):
+        for j in range(k):
+            ref = np.maximum(ref, z[:, :, i:i + h, j:j + w])
+    xd = torch.zeros(x.size + 8, dtype=torch.float16, device="cuda")
+    yd = torch.full((x.size + 8,), 7.0, dtype=torch.float16, device="cuda")
+    xd[off:off + x.size] = torch.from_numpy(x.reshape(-1)).cuda()
+    ops.pool(ops.POOL_MAX, xd[off:].data_ptr(), yd[off:].data_ptr(), c, h, w, k, 1, p, batch)
+    y = yd.cpu().numpy()
+    assert np.array_equal(y[off:off + x.size].reshape(x.shape), ref)
+    assert np.all(y[:off] == 7.0) and np.all(y[off + x.size:] == 7.0)
