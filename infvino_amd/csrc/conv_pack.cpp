@@ -41,6 +41,31 @@ float h2f_bits(uint16_t h)
   return f;
 }
 
+// fp32 [G][Cin/G][K][K][Cout/G], with room for the direct kernel's last 16-channel read
+size_t direct_bytes(const ConvSpec & s)
+{
+  return ((size_t)s.Cin * s.K * s.K * (s.Cout / s.G) + 32) * 4;
+}
+
+void pack_direct(const ConvSpec & s, const uint16_t * W, float * P)
+{
+  const int K2 = s.K * s.K, cin_g = s.Cin / s.G, cout_g = s.Cout / s.G;
+  for (int co = 0; co < s.Cout; ++co) {
+    const int g = co / cout_g, cl = co % cout_g;
+    for (int ci = 0; ci < cin_g; ++ci)
+      for (int t = 0; t < K2; ++t)
+        P[(((size_t)g * cin_g + ci) * K2 + t) * cout_g + cl] = h2f_bits(W[((size_t)co * cin_g + ci) * K2 + t]);
+  }
+}
+
+// 16-byte pieces of dense planes at every operand, images below the kernels' 2^31-byte buffers
+bool planes_vec_ok(const ConvParams & p)
+{
+  for (const View * v : {&p.x, &p.y, &p.r})
+    if (v->ptr && (reinterpret_cast<uintptr_t>(v->ptr) % 16 || v->img % 8 || v->img * 2 >= (1L << 31))) return false;
+  return true;
+}
+
 int halo_index(int ck) { return ck == 16 ? 0 : (ck == 32 ? 1 : 2); }
 
 }  // namespace
@@ -70,6 +95,7 @@ ConvPacking conv_packing(const ConvSpec & s)
     pk.cin8 = (int)rup(cin_g, 8);
     pk.kpad = igemm_kpad(s.Cout, s.K * s.K * pk.cin8);
     pk.w = seg((size_t)rows * pk.kpad * 2);
+    if (s.keep_direct) pk.direct = seg(direct_bytes(s));
     if (s.K == 3 && s.S == 1 && s.P == 1 && s.x_nhwc && !(s.flags & IVH_FLAG_NO_HALO)) {
       for (int cfg : {0, 7}) {  // every chunk size some tile config may use for this Cin
         const int ck = halo_cfg_ck(cfg, cin_g), hi = halo_index(ck);
@@ -94,7 +120,7 @@ ConvPacking conv_packing(const ConvSpec & s)
     pk.w = seg(((size_t)rows * 32 + 16 * 64) * 2);
     if (s.Cout <= 16) pk.stem_w2 = pk.w + (size_t)rows * 32 * 2;
   } else if (pk.family == kFamDirect) {
-    pk.w = seg(((size_t)s.G * cin_g * s.K * s.K * (s.Cout / s.G) + 32) * 4);
+    pk.w = seg(direct_bytes(s));
   } else {
     pk.w = seg(((size_t)s.K * s.K * s.Cout + 8) * 4);
     pk.dw_w16 = seg(((size_t)s.K * s.K * s.Cout + 8) * 2);
@@ -107,12 +133,13 @@ void conv_pack(const ConvSpec & s, const ConvPacking & pk, const uint16_t * W, c
                std::vector<uint8_t> & blob)
 {
   blob.assign(pk.bytes, 0);
-  const int Cout = s.Cout, K = s.K, G = s.G, cin_g = s.Cin / s.G;
+  const int Cout = s.Cout, K = s.K, cin_g = s.Cin / s.G;
   auto at = [&](int co, int ci, int t) { return W[((size_t)co * cin_g + ci) * K * K + t]; };
   if (pk.bias != kNoSeg) {
     float * bf = reinterpret_cast<float *>(blob.data() + pk.bias);
     for (int c = 0; c < Cout; ++c) bf[c] = B ? h2f_bits(B[c]) : 0.0f;
   }
+  if (pk.direct != kNoSeg) pack_direct(s, W, reinterpret_cast<float *>(blob.data() + pk.direct));
   if (pk.family == kFamIgemm) {
     uint16_t * P = reinterpret_cast<uint16_t *>(blob.data() + pk.w);
     for (int co = 0; co < Cout; ++co)
@@ -151,14 +178,7 @@ void conv_pack(const ConvSpec & s, const ConvPacking & pk, const uint16_t * W, c
           for (int t = 0; t < 9; ++t) P2[co * 64 + t * 4 + ci] = at(co, ci, t);
     }
   } else if (pk.family == kFamDirect) {
-    float * P = reinterpret_cast<float *>(blob.data() + pk.w);
-    const int cout_g = Cout / G;
-    for (int co = 0; co < Cout; ++co) {
-      const int g = co / cout_g, cl = co % cout_g;
-      for (int ci = 0; ci < cin_g; ++ci)
-        for (int t = 0; t < K * K; ++t)
-          P[(((size_t)g * cin_g + ci) * K * K + t) * cout_g + cl] = h2f_bits(at(co, ci, t));
-    }
+    pack_direct(s, W, reinterpret_cast<float *>(blob.data() + pk.w));
   } else {
     float * P = reinterpret_cast<float *>(blob.data() + pk.w);
     uint16_t * P16 = reinterpret_cast<uint16_t *>(blob.data() + pk.dw_w16);
@@ -183,6 +203,10 @@ int conv_resolve(const ConvSpec & s, const ConvPacking & pk, const void * dev_bl
   if (pk.family == kFamDirect) {
     p.stem_mfma = pk.stem ? 1 : 0;
     if (pk.stem && pk.stem_w2 != kNoSeg) p.w2 = reinterpret_cast<const __half *>(base + pk.stem_w2);
+    return kLaunchDirect;
+  }
+  if (pk.direct != kNoSeg && !planes_vec_ok(p)) {
+    p.w = reinterpret_cast<const __half *>(base + pk.direct);
     return kLaunchDirect;
   }
   p.cin8 = pk.cin8;

@@ -26,6 +26,8 @@ struct ConvSpec {
   bool x_vec1 = false;  // single-pixel NCHW input (an FC / GEMV): the MFMA family reads it too
   bool x_planes8 = false;  // 1x1 conv on NCHW input whose planes hold a multiple of 8 pixels:
                            // the MFMA family reads it, transposing pixel pieces in LDS
+  bool keep_direct = false;  // x_planes8 and the caller's pointers may lack 16-byte alignment:
+                             // the blob also holds the direct kernel's weights
   uint32_t flags = 0;   // IVH_FLAG_DIRECT_ONLY / IVH_FLAG_NO_HALO
   int Ho() const { return (H + 2 * P - K) / S + 1; }
   int Wo() const { return (W + 2 * P - K) / S + 1; }
@@ -38,6 +40,7 @@ struct ConvPacking {
   int family = kFamDirect;
   size_t bias = kNoSeg;              // fp32 [round_up(Cout, 128) + 16]
   size_t w = kNoSeg;                 // the family's main packing
+  size_t direct = kNoSeg;            // implicit GEMM with keep_direct: the direct kernel's fp32 weights too
   int cin8 = 0, kpad = 0;            // implicit GEMM: fp16 [round_up(Cout,128)][kpad]
   size_t halo[3] = {kNoSeg, kNoSeg, kNoSeg};  // 3x3 s1 p1: fp16 [rows][chunk][tap][ck], ck 16/32/64
   int kpad_halo[3] = {0, 0, 0};

@@ -226,3 +226,32 @@ def test_abi_maxpool_planes(k, c, h, w, batch, off):
     y = yd.cpu().numpy()
     assert np.array_equal(y[off:off + x.size].reshape(x.shape), ref)
     assert np.all(y[:off] == 7.0) and np.all(y[off + x.size:] == 7.0)
+
+
+@pytest.mark.parametrize("cin,cout,h,w,res,off", [
+    (9, 9, 2, 4, False, 0),       # the fewest pixels and channels of the MFMA route
+    (64, 128, 8, 8, False, 0),    # planar streaming kernel
+    (130, 140, 4, 10, True, 0),   # planar implicit GEMM: a K remainder, two channel tiles, residual
+    (24, 33, 6, 20, True, 1),     # pointers one element off a 16-byte boundary: the direct kernel
+    (24, 8, 6, 20, False, 0),     # up to 8 output channels, and ...
+    (24, 33, 5, 5, False, 0),     # ... planes of an odd size: the direct family
+])
+def test_abi_pointwise_planes(cin, cout, h, w, res, off):
+    B, n_in, n_out = 3, cin * h * w, cout * h * w
+    rng = np.random.default_rng(cin + cout)
+    d = ops.conv_desc(cin, cout, h, w, act=ops.ACT_SILU, channels_last=False)
+    x = O.f2h(rng.random(B * n_in).astype(np.float32))
+    wt = O.f2h((rng.standard_normal(cout * cin) * np.sqrt(2.0 / cin)).astype(np.float32))
+    bias = O.f2h((rng.standard_normal(cout) * 0.01).astype(np.float32))
+    r = O.f2h(rng.random(B * n_out).astype(np.float32)) if res else None
+    packed = _pack(d, wt, bias)
+    pad = lambda a: _dev(np.concatenate([np.full(off, NAN16, np.uint16), a, np.full(8, NAN16, np.uint16)]))
+    xd, yd, rd = pad(x), pad(np.full(B * n_out, NAN16, np.uint16)), pad(r) if res else None
+    ops.conv2d(d, xd[off:].data_ptr(), packed.data_ptr(), rd[off:].data_ptr() if res else None, yd[off:].data_ptr(), B)
+    y = _host(yd)
+    assert np.all(y[:off] == NAN16) and np.all(y[off + B * n_out:] == NAN16)
+    got = y[off:off + B * n_out].reshape(B, -1)
+    for b in range(B):
+        ref = O.conv2d(x[b * n_in:(b + 1) * n_in], wt, bias, None if r is None else r[b * n_out:(b + 1) * n_out],
+                       cin, h, w, cout, 1, 1, 0, 1, h, w, ops.ACT_SILU, O.F32, 2)
+        assert _ok(got[b], ref, f"planes {cin}->{cout} image {b}")
