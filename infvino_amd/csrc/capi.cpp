@@ -73,6 +73,7 @@ ivh::ConvSpec conv_spec(const ivh_conv_desc * d, bool gemv)
   s.has_bias = d->has_bias != 0;
   s.x_nhwc = d->channels_last != 0;
   s.x_vec1 = gemv && d->cin % 8 == 0;
+  s.lone = true;
   // 1x1 on planes of whole 8-pixel pieces, as the plan executor routes them: the MFMA kernels
   // (64->128 at 80x80, one image: 35.7 us a call on the direct kernel, 5.2 us).  Up to 8 output channels
   // the direct family's vector kernel, which is no slower, stays; so do odd planes and, from

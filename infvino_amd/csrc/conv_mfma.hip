@@ -442,6 +442,7 @@ ConvParams conv_batch_slice(const ConvParams & p, int b0, int nb)
 std::string igemm_launch_tag(const ConvParams & p)
 {
   char b[160];
+  if (p.small) return small_launch_tag(p);
   if (p.pw == 2)
     snprintf(b, sizeof b, "blocks=%ld lds=%zu planar-out%s", pw_blocks(p), pwt_lds_bytes(p), p.xt ? " planar-in" : "");
   else if (p.pw)
@@ -470,6 +471,10 @@ void launch_conv_igemm(const ConvParams & p, hipStream_t s)
   const int bc = conv_batch_chunk(p);
   if (bc < p.batch) {
     for (int b0 = 0; b0 < p.batch; b0 += bc) launch_conv_igemm(conv_batch_slice(p, b0, std::min(bc, p.batch - b0)), s);
+    return;
+  }
+  if (p.small) {
+    launch_conv_small(p, s);
     return;
   }
   if (p.pw) {

@@ -66,6 +66,21 @@ bool planes_vec_ok(const ConvParams & p)
   return true;
 }
 
+// the small-grid kernel where it is the faster one; not with NO_SPLITK, under which an image's
+// fp32 sums have one order at every batch size
+bool use_small(const ConvSpec & s, ConvParams & p)
+{
+  if (s.flags & (IVH_FLAG_NO_SPLITK | IVH_FLAG_PIPE_ANY)) return false;
+  // plans keep the resident-weight kernel for the 3x3 convs of 17..64 channels at every batch
+  // (their tests pin it); a lone call does not: 64->64 at 40x40, one image, 8.9 -> 4.4 us
+  if (!s.lone && p.K == 3 && p.S == 1 && p.Cin > 16 && p.Cin <= 64) return false;
+  p.small = small_plan(p);
+  if (!p.small) return false;
+  p.ksplit = 1;
+  p.ws = nullptr;
+  return true;
+}
+
 int halo_index(int ck) { return ck == 16 ? 0 : (ck == 32 ? 1 : 2); }
 
 }  // namespace
@@ -240,8 +255,11 @@ int conv_resolve(const ConvSpec & s, const ConvPacking & pk, const void * dev_bl
   // implicit GEMM, the one family with that input
   if (p.cu) {
     if (!upcat_ok(p)) throw std::runtime_error("upsample-concat input geometry");
+    use_small(s, p);
     return kLaunchIgemm;
   }
+  // grids too small for the chip: K split over the waves of a work-group
+  if (use_small(s, p)) return kLaunchIgemm;
   // 1x1 stride 1 with Cout <= 128 on channels-last views: the streaming pointwise kernel of
   // conv_pw.hip when its 32-pixel blocks fill the persistent grid several times over, and
   // where it was measured faster than the implicit GEMM (MI355X, batch 64, kernel trace):

@@ -28,6 +28,7 @@ struct ConvSpec {
                            // the MFMA family reads it, transposing pixel pieces in LDS
   bool keep_direct = false;  // x_planes8 and the caller's pointers may lack 16-byte alignment:
                              // the blob also holds the direct kernel's weights
+  bool lone = false;    // a single-op call, not a plan's node
   uint32_t flags = 0;   // IVH_FLAG_DIRECT_ONLY / IVH_FLAG_NO_HALO
   int Ho() const { return (H + 2 * P - K) / S + 1; }
   int Wo() const { return (W + 2 * P - K) / S + 1; }

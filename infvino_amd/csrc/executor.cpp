@@ -1662,7 +1662,7 @@ bool Model::pairLaunch(size_t ni, int batch, Launch & L)
   if (!pair_plan(C, b.H, b.W, batch, &th, &tw)) return false;
   b.th = th;
   b.tw = tw;
-  b.pipe = b.wide = b.res = b.halo = b.s2 = 0;
+  b.pipe = b.wide = b.res = b.halo = b.s2 = b.small = A.cp.small = 0;
   b.ksplit = 1;
   b.ws = nullptr;
   L.kind = Launch::kPair;
@@ -2301,6 +2301,12 @@ void Model::validate(const Launch & l) const
       }
       const long rows = (long)(p.Cout + igemm_bn(p.Cout) - 1) / igemm_bn(p.Cout) * igemm_bn(p.Cout);
       check(p.w, 0, rows * p.kpad - 1, 2, "igemm w");
+      if (p.small) {
+        if (p.small < 0 || p.small > kSmallCfgs || p.halo || p.res || p.pipe || p.wide || p.s2 || p.pw || p.ksplit != 1 ||
+            !small_views_ok(p))
+          throw std::runtime_error("small-grid conv geometry");
+        check(p.w, 0, (long)(p.Cout + 63) / 64 * 64 * p.kpad - 1, 2, "small-grid conv w");
+      }
       if (p.halo) {
         const int cfg = p.halo - 1, ck = p.ck;
         if (cfg < 0 || cfg >= kHaloCfgs || ck != halo_cfg_ck(cfg, p.Cin)) throw std::runtime_error("halo chunk size");
@@ -2794,7 +2800,7 @@ std::string Model::nodeKernel(int i)
   const Launch & l = P.L[P.begin[i]];
   switch (l.kind) {
   case Launch::kIgemm:
-    return l.cp.wide ? "conv_wide" : l.cp.pipe ? "conv_pipe" : l.cp.res ? "conv_res" : l.cp.halo ? "conv_halo" : (l.cp.pw == 2 ? "conv_pw_planar" : l.cp.pw ? "conv_pw" : l.cp.s2 ? (l.cp.s2 > 2 ? "conv_s2p" : "conv_s2") : (l.cp.ksplit > 1 ? "conv_igemm_sk" : "conv_igemm"));
+    return l.cp.wide ? "conv_wide" : l.cp.pipe ? "conv_pipe" : l.cp.res ? "conv_res" : l.cp.halo ? "conv_halo" : (l.cp.pw == 2 ? "conv_pw_planar" : l.cp.pw ? "conv_pw" : l.cp.s2 ? (l.cp.s2 > 2 ? "conv_s2p" : "conv_s2") : (l.cp.ksplit > 1 || l.cp.small ? "conv_igemm_sk" : "conv_igemm"));
   case Launch::kDirect: return l.cp.stem_mfma ? "conv_stem" : "conv_direct";
   case Launch::kDw: return "dwconv";
   case Launch::kDecode: return "pose_decode";

@@ -95,6 +95,9 @@ struct ConvParams {
   // 1x1 stride-1 streaming kernel (conv_pw.hip, Cout <= 64, channels-last views): 1 when
   // used; w is then the implicit-GEMM packing
   int pw = 0;
+  // small-grid implicit GEMM (conv_small.hip, K split over a work-group's waves): config + 1
+  // (0: not used); w is the implicit-GEMM packing
+  int small = 0;
   // implicit GEMM of a 1x1 conv reading NCHW channel planes (x.cs = pixels per plane, a
   // multiple of 8): each thread loads 8 consecutive pixels of one channel and writes them
   // transposed into the tile's pixel rows in LDS (0: channels-last input)

@@ -24,6 +24,15 @@ int conv_batch_chunk(const ConvParams & p);                      // images per l
 ConvParams conv_batch_slice(const ConvParams & p, int b0, int nb);  // images [b0, b0 + nb)
 int igemm_ksplit(long M, int cout, int kpad);  // 1 = no split
 
+// conv_small.hip: implicit GEMM whose K range is split over a work-group's waves, for grids
+// too small to fill the chip
+constexpr int kSmallCfgs = 4;
+int small_plan(const ConvParams & p);               // config + 1, 0: another kernel is faster or needed
+bool small_views_ok(const ConvParams & p);          // channels-last operands, 16-byte input pieces
+long small_grid(const ConvParams & p, int cfg);     // work-groups
+std::string small_launch_tag(const ConvParams & p);
+void launch_conv_small(const ConvParams & p, hipStream_t s);
+
 // conv_halo.hip: 3x3 stride-1 pad-1 convs with an LDS input patch
 constexpr int kHaloCfgs = 9;         // tile configs of the LDS-patch kernel
 int halo_cfg_ck(int cfg, int cin);  // input-channel chunk a tile config uses (16 / 32 / 64)

@@ -255,3 +255,38 @@ def test_abi_pointwise_planes(cin, cout, h, w, res, off):
         ref = O.conv2d(x[b * n_in:(b + 1) * n_in], wt, bias, None if r is None else r[b * n_out:(b + 1) * n_out],
                        cin, h, w, cout, 1, 1, 0, 1, h, w, ops.ACT_SILU, O.F32, 2)
         assert _ok(got[b], ref, f"planes {cin}->{cout} image {b}")
+
+
+@pytest.mark.parametrize("cin,cout,h,w,k,s,B,res", [
+    (256, 256, 20, 20, 3, 1, 1, False),   # 32 x 32 tiles, eight waves of nine chunks
+    (128, 100, 13, 11, 3, 2, 2, True),    # the same with uneven K shares, ragged channels, residual
+    (40, 33, 7, 9, 1, 1, 1, False),       # 32 x 32 tiles, four waves, the last ones without work
+    (21, 19, 5, 5, 3, 1, 1, True),        # Cin % 8: chunks of four pieces straddle taps, masked tails
+    (8, 12, 6, 6, 5, 1, 3, False),        # four taps a chunk
+    (128, 192, 40, 40, 3, 1, 1, True),    # 64 x 32 tiles, eight waves
+    (64, 64, 40, 40, 3, 1, 8, True),      # 64 x 64 tiles, pixels of two images in a tile
+    (60, 130, 39, 39, 1, 1, 3, False),    # the same with a half-empty last channel tile, Cin % 8
+    (256, 64, 3, 3, 1, 2, 5, False),      # stride 2 pointwise
+])
+def test_abi_small_grid_conv(cin, cout, h, w, k, s, B, res):
+    """Convs of few pixels (K split over a work-group's waves) at the edges of its tiles."""
+    p, act = k // 2, ops.ACT_SILU
+    rng = np.random.default_rng(cin * 7 + cout)
+    d = ops.conv_desc(cin, cout, h, w, k, s, p, act=act)
+    ho, wo = ops.conv_out_dims(d)
+    x = O.f2h((rng.random(B * cin * h * w) * 2 - 1).astype(np.float32))
+    wt = O.f2h((rng.standard_normal(cout * cin * k * k) * np.sqrt(2.0 / (cin * k * k))).astype(np.float32))
+    bias = O.f2h((rng.standard_normal(cout) * 0.1).astype(np.float32))
+    r = O.f2h(rng.random(B * cout * ho * wo).astype(np.float32)) if res else None
+    packed = _pack(d, wt, bias)
+    xd, rd = _dev(_nhwc(x, B, cin, h, w)), _dev(_nhwc(r, B, cout, ho, wo)) if res else None
+    yd = _dev(np.full(B * ho * wo * ((cout + 7) // 8 * 8) + 64, NAN16, np.uint16))
+    ops.conv2d(d, xd.data_ptr(), packed.data_ptr(), rd.data_ptr() if res else None, yd.data_ptr(), B)
+    y = _host(yd)
+    assert np.all(y[-64:] == NAN16)
+    got = _from_nhwc(y[:-64], B, cout, ho, wo)
+    for b in range(B):
+        ref = O.conv2d(x[b * cin * h * w:(b + 1) * cin * h * w], wt, bias,
+                       None if r is None else r[b * cout * ho * wo:(b + 1) * cout * ho * wo],
+                       cin, h, w, cout, k, s, p, 1, ho, wo, act, O.F32, 2)
+        assert _ok(got[b], ref, f"small-grid conv {cin}->{cout} k{k} s{s} image {b}")
