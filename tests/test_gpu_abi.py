@@ -290,3 +290,25 @@ def test_abi_small_grid_conv(cin, cout, h, w, k, s, B, res):
                        None if r is None else r[b * cout * ho * wo:(b + 1) * cout * ho * wo],
                        cin, h, w, cout, k, s, p, 1, ho, wo, act, O.F32, 2)
         assert _ok(got[b], ref, f"small-grid conv {cin}->{cout} k{k} s{s} image {b}")
+
+
+@pytest.mark.parametrize("bb,m,k,n,batch", [
+    (1, 1, 1, 1, 1), (2, 65, 63, 129, 2), (3, 49, 64, 49, 1), (1, 130, 70, 64, 3), (2, 33, 201, 17, 2),
+    (1, 128, 128, 128, 1), (2, 8, 65, 65, 5),
+])
+def test_abi_bmm_edges(bb, m, k, n, batch):
+    """Both tile shapes (N up to 64 and above) at odd row lengths, K remainders and partial tiles."""
+    rng = np.random.default_rng(m * n + k)
+    L = O.lib()
+    a = O.f2h((rng.standard_normal(batch * bb * m * k) * 0.5).astype(np.float32))
+    bm = O.f2h((rng.standard_normal(batch * bb * k * n) * 0.5).astype(np.float32))
+    ad, bd = _dev(a), _dev(bm)
+    yd = _dev(np.full(batch * bb * m * n + 16, NAN16, np.uint16))
+    ops.bmm(ad.data_ptr(), bd.data_ptr(), yd.data_ptr(), bb, m, k, n, batch)
+    y = _host(yd)
+    assert np.all(y[-16:] == NAN16)
+    got = y[:-16].reshape(batch, -1)
+    for b in range(batch):
+        ref = np.empty(bb * m * n, np.uint16)
+        L.ivo_bmm(a[b * bb * m * k:(b + 1) * bb * m * k], bm[b * bb * k * n:(b + 1) * bb * k * n], ref, bb, m, k, n)
+        assert _ok(got[b], ref, f"bmm {bb}x{m}x{k}x{n} image {b}")
