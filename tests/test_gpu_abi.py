@@ -312,3 +312,26 @@ def test_abi_bmm_edges(bb, m, k, n, batch):
         ref = np.empty(bb * m * n, np.uint16)
         L.ivo_bmm(a[b * bb * m * k:(b + 1) * bb * m * k], bm[b * bb * k * n:(b + 1) * bb * k * n], ref, bb, m, k, n)
         assert _ok(got[b], ref, f"bmm {bb}x{m}x{k}x{n} image {b}")
+
+
+@pytest.mark.parametrize("axis", [1, 7, 8, 63, 64, 65, 128, 129, 256, 399, 512, 513, 1024, 2047, 2048, 2049])
+def test_abi_softmax_rows(axis):
+    """Rows of every lane count and piece count, at odd offsets, with a masked (-inf), a lowest
+    (-65504), an all-equal and a large row."""
+    rng = np.random.default_rng(axis)
+    L, outer = O.lib(), 37
+    v = (rng.standard_normal((outer, axis)) * 3).astype(np.float32)
+    v[1, : axis // 2] = -np.inf
+    v[2, axis // 3:] = -65504
+    v[3] = 65504
+    v[4] = -65504
+    s = O.f2h(v.ravel())
+    sd = torch.zeros(s.size + 1, dtype=torch.int16, device="cuda")
+    sd[1:] = _dev(s)
+    od = _dev(np.full(s.size + 17, NAN16, np.uint16))
+    ops.softmax(sd[1:].data_ptr(), od[1:].data_ptr(), outer, axis, 1, 1)
+    y = _host(od)
+    assert y[0] == NAN16 and np.all(y[1 + s.size:] == NAN16)
+    ref = np.empty(s.size, np.uint16)
+    L.ivo_softmax_axis(s, ref, outer, axis, 1)
+    assert _ok(y[1:1 + s.size], ref, f"softmax rows of {axis}")
