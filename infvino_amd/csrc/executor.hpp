@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <functional>
 #include <map>
 #include <memory>
 #include <string>
@@ -167,6 +168,15 @@ class Model {
   void * arena_ = nullptr;                  // activations, max_batch images
   long arena_elems1_ = 0;                   // elements per image-unit
   void * input_buf_ = nullptr;              // graph input, max_batch images (fp16)
+  // Readback through pinned host memory: a ring of kRingSlots chunks, allocated by the first
+  // read that needs it and given back with the model
+  static constexpr int kRingSlots = 16, kRingThreads = 8;
+  static constexpr size_t kRingChunk = 1 << 20;
+  char * ring_ = nullptr;
+  hipEvent_t ring_ev_[kRingSlots] = {};
+  bool ringReady();
+  // `dst[0, bytes)` from chunks that fill(pinned chunk, offset, bytes) enqueues on the stream
+  void ringRead(char * dst, size_t bytes, const std::function<void(char *, size_t, size_t)> & fill);
   void * stage_f32_ = nullptr;              // f32 staging for the truncating conversion
   std::vector<void *> dev_allocs_;          // weights etc.
   size_t weight_bytes_ = 0;

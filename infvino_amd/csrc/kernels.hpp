@@ -163,6 +163,8 @@ constexpr long kBoundaryScratchFloats = 1L << 21;
 float * boundary_scratch(int device);
 // one mutex per device, held by a caller while its copies and kernels use that device's array
 std::mutex & boundary_scratch_lock(int device);
+// device memory to pinned host memory by a kernel (bytes % 2 == 0)
+void launch_copy_out(const void * in, void * out, long bytes, hipStream_t s);
 void launch_f16_to_f32(const __half * in, float * out, long n, hipStream_t s);
 
 }  // namespace ivh

@@ -2075,11 +2075,42 @@ __global__ void f32_to_f16_trunc_kernel(const float * in, uint16_t * out, long n
   out[i] = (uint16_t)h;
 }
 
-__global__ void f16_to_f32_kernel(const __half * in, float * out, long n)
+// Exact f16 -> f32, NaN payloads included (the conversion instruction would quieten signalling
+// ones).  `out` is pinned host memory in the readback path: a lane writes 16 consecutive
+// bytes, a wave 1 KB, so the writes cross PCIe as whole bursts.
+__global__ void __launch_bounds__(256) f16_to_f32_kernel(const __half * in, float * out, long n)
 {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= n) return;
-  out[i] = (float)reinterpret_cast<const _Float16 *>(in)[i];
+  typedef unsigned short u16x4u __attribute__((ext_vector_type(4), aligned(2)));
+  typedef unsigned u32x4u __attribute__((ext_vector_type(4), aligned(4)));
+  const unsigned short * src = reinterpret_cast<const unsigned short *>(in);
+  auto cvt = [](unsigned short h) {
+    const unsigned inf_nan = ((unsigned)(h & 0x8000u) << 16) | 0x7f800000u | ((unsigned)(h & 0x3ffu) << 13);
+    return (h & 0x7c00u) == 0x7c00u ? inf_nan : __builtin_bit_cast(unsigned, (float)__builtin_bit_cast(_Float16, h));
+  };
+  if (i + 4 <= n) {
+    const u16x4u v = *reinterpret_cast<const u16x4u *>(src + i);
+    *reinterpret_cast<u32x4u *>(out + i) = u32x4u{cvt(v[0]), cvt(v[1]), cvt(v[2]), cvt(v[3])};
+  } else {
+    for (long k = i; k < n; ++k) reinterpret_cast<unsigned *>(out)[k] = cvt(src[k]);
+  }
+}
+
+// n bytes (a multiple of 2) to pinned host memory, 16 a lane
+__global__ void __launch_bounds__(256) copy_out_kernel(const char * in, char * out, long n)
+{
+  const long i = ((long)blockIdx.x * 256 + threadIdx.x) * 16;
+  if (i + 16 <= n) {
+    *reinterpret_cast<h8u *>(out + i) = *reinterpret_cast<const h8u *>(in + i);
+  } else {
+    for (long k = i; k < n; k += 2) *reinterpret_cast<short *>(out + k) = *reinterpret_cast<const short *>(in + k);
+  }
+}
+void launch_copy_out(const void * in, void * out, long bytes, hipStream_t s)
+{
+  hipLaunchKernelGGL(copy_out_kernel, dim3(nblk(bytes, 4096)), dim3(256), 0, s, static_cast<const char *>(in),
+                     static_cast<char *>(out), bytes);
 }
 
 void launch_f32_to_f16_trunc(const float * in, __half * out, long n, hipStream_t s)
@@ -2131,7 +2162,7 @@ float * boundary_scratch(int device)
 
 void launch_f16_to_f32(const __half * in, float * out, long n, hipStream_t s)
 {
-  hipLaunchKernelGGL(f16_to_f32_kernel, dim3(nblk(n, 256)), dim3(256), 0, s, in, out, n);
+  hipLaunchKernelGGL(f16_to_f32_kernel, dim3(nblk(n, 1024)), dim3(256), 0, s, in, out, n);
 }
 
 }  // namespace ivh

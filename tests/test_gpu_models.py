@@ -354,3 +354,22 @@ def test_profiling_mode_accumulates(tmp_path):
     assert ia.lib().ivh_node_times(m._h, ms, calls, n) == 0
     assert sum(calls) == 0
     m.close()
+
+
+@pytest.mark.parametrize("hw,batch", [(8, 1), (725, 1), (1200, 1), (1024, 5), (1100, 40)])
+def test_readback_sizes(tmp_path, hw, batch):
+    """Outputs read as fp16 and f32 through the pinned ring: part of a chunk, several chunks
+    with an odd tail, and more chunks than slots on several threads; every half pattern among
+    the values, the floats exact (NaN payloads included)."""
+    n = hw * hw
+    path = tmp_path / "io.plan"
+    path.write_text(f"input x 1 1 {hw} {hw}\ntensor y 1 1 {hw} {hw}\nnode copy_c x y HW={n} c0=0 cnt=1 dst_off=0\noutput y\n")
+    m = ia.PlanModel(str(path), 0, batch, ia.IVH_FLAG_NO_FUSE)
+    x = np.resize(np.arange(65536, dtype=np.uint16), n * batch) ^ np.uint16(batch)
+    m.setInput(x, batch)
+    m.run(batch)
+    for _ in range(2):  # the second read reuses the ring
+        assert np.array_equal(m.readOutput(0, batch), x)
+        f = m.readOutputF32(0, batch)
+        assert np.array_equal(f.view(np.uint32), O.h2f(x).view(np.uint32))
+    m.close()
