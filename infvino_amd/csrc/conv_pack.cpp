@@ -81,6 +81,15 @@ bool use_small(const ConvSpec & s, ConvParams & p)
   return true;
 }
 
+// the DMA-fed build of the implicit GEMM where it is the faster one
+void use_ring(const ConvSpec & s, ConvParams & p)
+{
+  p.ring = ring_plan(p, (s.flags & IVH_FLAG_NO_SPLITK) != 0);
+  if (!p.ring) return;
+  p.ksplit = 1;
+  p.ws = nullptr;
+}
+
 int halo_index(int ck) { return ck == 16 ? 0 : (ck == 32 ? 1 : 2); }
 
 }  // namespace
@@ -255,7 +264,7 @@ int conv_resolve(const ConvSpec & s, const ConvPacking & pk, const void * dev_bl
   // implicit GEMM, the one family with that input
   if (p.cu) {
     if (!upcat_ok(p)) throw std::runtime_error("upsample-concat input geometry");
-    use_small(s, p);
+    if (!use_small(s, p)) use_ring(s, p);
     return kLaunchIgemm;
   }
   // grids too small for the chip: K split over the waves of a work-group
@@ -424,7 +433,7 @@ int conv_resolve(const ConvSpec & s, const ConvPacking & pk, const void * dev_bl
   if (p.x.layout != kNHWC || (p.x.cs % 8) || (p.x.img % 8) || (reinterpret_cast<uintptr_t>(p.x.ptr) % 16))
     throw std::runtime_error("implicit-GEMM input view not 16-byte aligned NHWC");
   if (p.kpad < p.K * p.K * p.cin8 || p.cin8 < p.Cin) throw std::runtime_error("packed weight geometry");
-  (void)s;
+  if (!p.halo && !p.s2) use_ring(s, p);
   return kLaunchIgemm;
 }
 

@@ -30,6 +30,9 @@ typedef __attribute__((address_space(3))) void lds_void;
 // 64 lanes x 16 bytes from a buffer to consecutive LDS pieces at `lds` (wave uniform)
 __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, _Float16 * lds, unsigned voff)
 {
+  // the offset is computed here for every lane: left to itself the compiler splits a copy into
+  // one for the lanes inside the image and one for the others
+  __asm__ volatile("" : "+v"(voff));
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)lds, 16, (int)voff, 0, 0, 0);
 }
 }  // namespace

@@ -1666,7 +1666,7 @@ bool Model::pairLaunch(size_t ni, int batch, Launch & L)
   if (!pair_plan(C, b.H, b.W, batch, &th, &tw)) return false;
   b.th = th;
   b.tw = tw;
-  b.pipe = b.wide = b.res = b.halo = b.s2 = b.small = A.cp.small = 0;
+  b.pipe = b.wide = b.res = b.halo = b.s2 = b.small = b.ring = A.cp.small = A.cp.ring = 0;
   b.ksplit = 1;
   b.ws = nullptr;
   L.kind = Launch::kPair;
@@ -2311,6 +2311,8 @@ void Model::validate(const Launch & l) const
           throw std::runtime_error("small-grid conv geometry");
         check(p.w, 0, (long)(p.Cout + 63) / 64 * 64 * p.kpad - 1, 2, "small-grid conv w");
       }
+      if (p.ring && (p.ring > 2 || p.small || p.halo || p.res || p.pipe || p.wide || p.s2 || p.pw || p.ksplit != 1 || !ring_ok(p)))
+        throw std::runtime_error("DMA-fed implicit-GEMM geometry");
       if (p.halo) {
         const int cfg = p.halo - 1, ck = p.ck;
         if (cfg < 0 || cfg >= kHaloCfgs || ck != halo_cfg_ck(cfg, p.Cin)) throw std::runtime_error("halo chunk size");

@@ -33,6 +33,11 @@ long small_grid(const ConvParams & p, int cfg);     // work-groups
 std::string small_launch_tag(const ConvParams & p);
 void launch_conv_small(const ConvParams & p, hipStream_t s);
 
+// conv_ring.hip: the implicit GEMM fed by LDS DMA (channels-last, whole 8-channel pieces)
+bool ring_ok(const ConvParams & p);
+int ring_plan(const ConvParams & p, bool one_order);  // 0: conv_igemm_kernel, 1: whole K, 2: K halves
+void launch_conv_ring(const ConvParams & p, hipStream_t s);
+
 // conv_halo.hip: 3x3 stride-1 pad-1 convs with an LDS input patch
 constexpr int kHaloCfgs = 9;         // tile configs of the LDS-patch kernel
 int halo_cfg_ck(int cfg, int cin);  // input-channel chunk a tile config uses (16 / 32 / 64)

@@ -335,3 +335,43 @@ def test_abi_softmax_rows(axis):
     ref = np.empty(s.size, np.uint16)
     L.ivo_softmax_axis(s, ref, outer, axis, 1)
     assert _ok(y[1:1 + s.size], ref, f"softmax rows of {axis}")
+
+
+@pytest.mark.parametrize("cin,cout,h,w,k,s,B,res", [
+    (256, 128, 40, 40, 1, 1, 8, True),    # K halves of four steps, 128-channel tiles, residual
+    (72, 200, 29, 31, 3, 2, 40, False),   # an odd step count over the halves, partial tiles both ways
+    (64, 64, 80, 80, 3, 2, 8, False),     # 64-channel tiles
+    (264, 40, 33, 35, 1, 1, 20, True),    # the same, 9 steps, 40 of 64 channels
+    (40, 256, 53, 53, 1, 1, 7, False),    # whole K: two steps, the second ragged
+    (32, 136, 61, 59, 3, 2, 40, True),    # whole K with taps, a second channel tile of 8
+])
+def test_abi_dma_implicit_gemm(cin, cout, h, w, k, s, B, res):
+    """Implicit-GEMM convs through the DMA-fed kernel: image 0 and the last one against the oracle,
+    and every image equal to the same image at another place of the batch."""
+    p, act = k // 2, ops.ACT_SILU
+    rng = np.random.default_rng(cin * 7 + cout)
+    d = ops.conv_desc(cin, cout, h, w, k, s, p, act=act)
+    ho, wo = ops.conv_out_dims(d)
+    x = O.f2h((rng.random(B * cin * h * w) * 2 - 1).astype(np.float32))
+    wt = O.f2h((rng.standard_normal(cout * cin * k * k) * np.sqrt(2.0 / (cin * k * k))).astype(np.float32))
+    bias = O.f2h((rng.standard_normal(cout) * 0.1).astype(np.float32))
+    r = O.f2h(rng.random(B * cout * ho * wo).astype(np.float32)) if res else None
+    packed = _pack(d, wt, bias)
+    n = B * ho * wo * cout
+
+    def run(shift):
+        roll = lambda a: None if a is None else np.roll(a.reshape(B, -1), shift, axis=0).ravel()
+        xd, rd = _dev(_nhwc(roll(x), B, cin, h, w)), _dev(_nhwc(roll(r), B, cout, ho, wo)) if res else None
+        yd = _dev(np.full(n + 64, NAN16, np.uint16))
+        ops.conv2d(d, xd.data_ptr(), packed.data_ptr(), rd.data_ptr() if res else None, yd.data_ptr(), B)
+        y = _host(yd)
+        assert np.all(y[n:] == NAN16)
+        return np.roll(_from_nhwc(y[:n], B, cout, ho, wo), -shift, axis=0)
+
+    got = run(0)
+    assert np.array_equal(got, run(3))
+    for b in (0, B - 1):
+        ref = O.conv2d(x[b * cin * h * w:(b + 1) * cin * h * w], wt, bias,
+                       None if r is None else r[b * cout * ho * wo:(b + 1) * cout * ho * wo],
+                       cin, h, w, cout, k, s, p, 1, ho, wo, act, O.F32, 2)
+        assert _ok(got[b], ref, f"DMA implicit GEMM {cin}->{cout} k{k} s{s} image {b}")
