@@ -4,7 +4,7 @@
 //   LDS patch      fp16 [round_up(Cout,128)][chunk][tap][ck] (3x3 stride 1 pad 1)
 //   stem           fp16 [ceil(Cout/16)*16][32], k = ci*9 + tap; and [16][64], k = tap*4 + ci
 //   direct         fp32 [G][Cin/G][K][K][Cout/G]
-//   depthwise      fp32 [K][K][C]
+//   depthwise      fp32 [K][K][C], and fp16 [K][K][round_up(C, 8)]
 // (the reference packs per kernel too: PlanModel.cpp:232-334).
 #include "conv_pack.hpp"
 
@@ -147,7 +147,7 @@ ConvPacking conv_packing(const ConvSpec & s)
     pk.w = seg(direct_bytes(s));
   } else {
     pk.w = seg(((size_t)s.K * s.K * s.Cout + 8) * 4);
-    pk.dw_w16 = seg(((size_t)s.K * s.K * s.Cout + 8) * 2);
+    pk.dw_w16 = seg((size_t)s.K * s.K * rup(s.Cout, 8) * 2);
   }
   pk.bytes = off;
   return pk;
@@ -206,10 +206,11 @@ void conv_pack(const ConvSpec & s, const ConvPacking & pk, const uint16_t * W, c
   } else {
     float * P = reinterpret_cast<float *>(blob.data() + pk.w);
     uint16_t * P16 = reinterpret_cast<uint16_t *>(blob.data() + pk.dw_w16);
+    const size_t c8 = (size_t)rup(Cout, 8);
     for (int c = 0; c < Cout; ++c)
       for (int t = 0; t < K * K; ++t) {
         P[(size_t)t * Cout + c] = h2f_bits(W[(size_t)c * K * K + t]);
-        P16[(size_t)t * Cout + c] = W[(size_t)c * K * K + t];
+        P16[t * c8 + c] = W[(size_t)c * K * K + t];
       }
   }
 }

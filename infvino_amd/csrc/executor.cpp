@@ -2417,9 +2417,12 @@ void Model::validate(const Launch & l) const
       check(p.x.ptr, 0, vlast(p.x, p.batch, p.Cin, HW), 2, "direct x");
       check(p.w, 0, (long)p.Cin * p.K * p.K * (p.Cout / p.G) + 16 - 1, 4, "direct w");
     } else {
-      check(p.x.ptr, 0, vlast(p.x, p.batch, p.Cin, HW), 2, "dw x");
+      // the channels-last kernels read whole 8-channel pieces
+      const long c8 = dwconv_vectorizable(p) ? (p.Cin + 7) / 8 * 8 : p.Cin;
+      check(p.x.ptr, 0, vlast(p.x, p.batch, c8, HW), 2, "dw x");
+      if (p.r.ptr) check(p.r.ptr, 0, vlast(p.r, p.batch, c8, HWo), 2, "dw residual");
       check(p.w, 0, (long)p.K * p.K * p.Cin - 1, 4, "dw w");
-      check(p.w2, 0, (long)p.K * p.K * p.Cin - 1, 2, "dw w16");
+      check(p.w2, 0, (long)p.K * p.K * c8 - 1, 2, "dw w16");
     }
     return;
   }

@@ -471,6 +471,19 @@ constexpr int kDwMaxIt = 16;
 constexpr int kDwBufPieces = kDwMaxIt * 256;
 constexpr int kDwMaxW = 4;  // weight pieces per lane: K*K*G <= 1024
 
+// Eight channels of a pixel, or the first n of a last piece past which the channels belong to no
+// output of this conv.  (Its inputs there, padding that may hold anything, reach only them.)
+__device__ __forceinline__ void dw_store(_Float16 * y, const h8 & v, int n)
+{
+  if (n >= 8) {
+    *reinterpret_cast<h8 *>(y) = v;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 7; ++e)
+      if (e < n) y[e] = v[e];
+  }
+}
+
 template <int K, int S, int PX, int PY, int ACT>
 __global__ void __launch_bounds__(256) dw_tile_kernel(const ConvParams p, const DwTile t)
 {
@@ -488,10 +501,11 @@ __global__ void __launch_bounds__(256) dw_tile_kernel(const ConvParams p, const 
   const int ox0 = tx * t.BX * PX, oy0 = ty * t.BY * PY;
   const int ix0 = ox0 * S - p.P, iy0 = oy0 * S - p.P, c0 = tc * G * 8;
 
-  // this image's input view from channel c0 on, up to its last element
+  // this image's input view from channel c0 on, up to its last pixel's last 8-channel piece
+  const int C8 = (p.Cin + 7) >> 3;
   const __half * xb = p.x.ptr + (long)b * p.x.img + c0;
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<__half *>(xb), (short)0, (int)((((long)p.H * p.W - 1) * p.x.cs + p.Cin - c0) * 2), kBufDword3);
+      const_cast<__half *>(xb), (short)0, (int)((((long)p.H * p.W - 1) * p.x.cs + C8 * 8 - c0) * 2), kBufDword3);
   const h8 * wg = reinterpret_cast<const h8 *>(p.w2) + tc * G;
   h8 * const xs = reinterpret_cast<h8 *>(dw_lds);  // [IH][IW][G] window pieces, then [K*K][G] weights
   // window piece i = tid + 256 u: row i / RP of the window, piece rem = i % RP of that row
@@ -532,7 +546,7 @@ __global__ void __launch_bounds__(256) dw_tile_kernel(const ConvParams p, const 
     const int i = tid + u * 256;
     if (i < nw) {
       const int tap = idiv_small(i, G, inv_g);
-      wv[u] = wg[(int)__umul24(tap, p.Cin >> 3) + i - (int)__umul24(tap, G)];
+      wv[u] = wg[(int)__umul24(tap, C8) + i - (int)__umul24(tap, G)];
     }
   }
 #pragma unroll
@@ -605,7 +619,7 @@ __global__ void __launch_bounds__(256) dw_tile_kernel(const ConvParams p, const 
 #pragma unroll
         for (int e = 0; e < 8; ++e) out[e] = (_Float16)((float)out[e] + (float)rv[e]);
       }
-      *reinterpret_cast<h8 *>(yb + hw * p.y.cs) = out;
+      dw_store(yb + hw * p.y.cs, out, p.Cin - c);
     }
   }
 }
@@ -622,7 +636,7 @@ __global__ void __launch_bounds__(256) dw_strip_kernel(const ConvParams p, FastD
   // lane = (8-channel group, strip of PX output pixels of one row), channel groups fastest so
   // that neighbouring lanes read and write neighbouring 16-byte pieces
   constexpr int NX = (PX - 1) * S + K;  // input columns of a strip
-  const int C8 = p.Cin >> 3, nstrip = (p.Wo + PX - 1) / PX;
+  const int C8 = (p.Cin + 7) >> 3, nstrip = (p.Wo + PX - 1) / PX;
   const unsigned idx = blockIdx.x * 256u + threadIdx.x;
   const unsigned q = fastdiv(idx, d_c8), rowi = fastdiv(q, d_strip), b = fastdiv(rowi, d_ho);
   if (b >= (unsigned)p.batch) return;
@@ -648,7 +662,7 @@ __global__ void __launch_bounds__(256) dw_strip_kernel(const ConvParams p, FastD
     }
 #pragma unroll
     for (int kx = 0; kx < K; ++kx) {
-      const h8 wv = *reinterpret_cast<const h8 *>(W + (ky * K + kx) * p.Cin);
+      const h8 wv = *reinterpret_cast<const h8 *>(W + (ky * K + kx) * (C8 * 8));
 #pragma unroll
       for (int j = 0; j < PX; ++j) {
         const h8 v = xv[j * S + kx];
@@ -678,7 +692,7 @@ __global__ void __launch_bounds__(256) dw_strip_kernel(const ConvParams p, FastD
 #pragma unroll
       for (int e = 0; e < 8; ++e) out[e] = (_Float16)((float)out[e] + (float)rv[e]);
     }
-    *reinterpret_cast<h8 *>(yb + hw * p.y.cs) = out;
+    dw_store(yb + hw * p.y.cs, out, p.Cin - c);
   }
 }
 
@@ -759,15 +773,19 @@ __global__ void __launch_bounds__(256) dw_nchw_kernel(const ConvParams p, FastDi
   }
 }
 
+// Channels-last views of 16-byte pieces, any channel count: a last piece of fewer than
+// eight channels is computed whole and stored in part (145 channels 5x5 stride 2 at 107x107,
+// batch 16: 26 us; the any-layout kernel, one lane per pixel of one channel with its pixels a
+// whole channels-last row apart, takes 667 us).
 bool dwconv_vectorizable(const ConvParams & p)
 {
   auto al = [](const View & v) {
     return v.layout == kNHWC && ((v.cs | (int)v.img | (int)(reinterpret_cast<uintptr_t>(v.ptr) >> 1)) & 7) == 0;
   };
-  return p.w2 && (reinterpret_cast<uintptr_t>(p.w2) & 15) == 0 && (p.Cin % 8) == 0 && (p.K == 3 || p.K == 5) &&
+  return p.w2 && (reinterpret_cast<uintptr_t>(p.w2) & 15) == 0 && (p.K == 3 || p.K == 5) &&
          (p.S == 1 || p.S == 2) && al(p.x) && al(p.y) &&
-         (!p.r.ptr || al(p.r)) && (long)p.batch * p.Ho * p.Wo * (p.Cin / 8) < (1L << 31) &&
-         (((long)p.H * p.W - 1) * p.x.cs + p.Cin) * 2 < (1L << 31) &&  // one image's buffer range
+         (!p.r.ptr || al(p.r)) && (long)p.batch * p.Ho * p.Wo * ((p.Cin + 7) / 8) < (1L << 31) &&
+         (((long)p.H * p.W - 1) * p.x.cs + p.Cin + 7) * 2 < (1L << 31) &&  // one image's buffer range
          (long)p.H * p.W < (1L << 24);
 }
 
@@ -790,7 +808,7 @@ struct DwPick {
 
 static DwPick dw_pick_search(const ConvParams & p)
 {
-  const int C8 = p.Cin / 8, K = p.K, S = p.S;
+  const int C8 = (p.Cin + 7) / 8, K = p.K, S = p.S;
   const double hbm = (double)p.batch * ((double)p.H * p.W + (double)p.Ho * p.Wo) * p.Cin * 2.0;
   constexpr double kEnoughWaves = 2.5 * 1024;
   DwPick best;
@@ -892,15 +910,16 @@ static void launch_dw_strip(const ConvParams & p, hipStream_t s)
 {
   constexpr int PX = 4;
   const int nstrip = (p.Wo + PX - 1) / PX;
-  const long n = (long)p.batch * p.Ho * nstrip * (p.Cin / 8);
+  const int C8 = (p.Cin + 7) / 8;
+  const long n = (long)p.batch * p.Ho * nstrip * C8;
   hipLaunchKernelGGL((dw_strip_kernel<5, 2, PX, ACT>), dim3(nblk(n, 256)), dim3(256), 0, s, p,
-                     fastdiv_make((unsigned)(p.Cin / 8)), fastdiv_make((unsigned)nstrip), fastdiv_make((unsigned)p.Ho));
+                     fastdiv_make((unsigned)C8), fastdiv_make((unsigned)nstrip), fastdiv_make((unsigned)p.Ho));
 }
 
 // The strip kernel is taken for 5x5 stride 2 once it has at least 1.5 waves per SIMD.
 static bool dw_use_strip(const ConvParams & p)
 {
-  return p.K == 5 && p.S == 2 && (long)p.batch * p.Ho * ((p.Wo + 3) / 4) * (p.Cin / 8) >= 1536L * 64;
+  return p.K == 5 && p.S == 2 && (long)p.batch * p.Ho * ((p.Wo + 3) / 4) * ((p.Cin + 7) / 8) >= 1536L * 64;
 }
 
 std::string dw_launch_tag(const ConvParams & p)

@@ -375,3 +375,33 @@ def test_abi_dma_implicit_gemm(cin, cout, h, w, k, s, B, res):
                        None if r is None else r[b * cout * ho * wo:(b + 1) * cout * ho * wo],
                        cin, h, w, cout, k, s, p, 1, ho, wo, act, O.F32, 2)
         assert _ok(got[b], ref, f"DMA implicit GEMM {cin}->{cout} k{k} s{s} image {b}")
+
+
+@pytest.mark.parametrize("c,h,w,k,s,B,res", [
+    (2, 5, 5, 3, 1, 2, False), (7, 9, 11, 5, 2, 1, True), (9, 14, 14, 3, 2, 3, False), (51, 20, 20, 3, 1, 4, True),
+    (145, 13, 17, 5, 1, 2, False), (70, 28, 28, 5, 2, 256, False), (33, 112, 112, 3, 1, 2, False),
+])
+def test_abi_depthwise_ragged_channels(c, h, w, k, s, B, res):
+    """Depthwise convs whose channel count leaves a partial last piece (tile and strip kernels):
+    NaN in the padding channels reaches no output, and the output's own padding stays."""
+    p, act = k // 2, ops.ACT_HSWISH
+    rng = np.random.default_rng(c * 10 + k)
+    d = ops.conv_desc(c, c, h, w, k, s, p, c, act)
+    ho, wo = ops.conv_out_dims(d)
+    x = O.f2h((rng.random(B * c * h * w) * 2 - 1).astype(np.float32))
+    wt = O.f2h((rng.standard_normal(c * k * k) * np.sqrt(2.0 / (k * k))).astype(np.float32))
+    bias = O.f2h((rng.standard_normal(c) * 0.1).astype(np.float32))
+    r = O.f2h(rng.random(B * c * ho * wo).astype(np.float32)) if res else None
+    packed = _pack(d, wt, bias)
+    xd, rd = _dev(_nhwc(x, B, c, h, w)), _dev(_nhwc(r, B, c, ho, wo)) if res else None
+    c8 = (c + 7) // 8 * 8
+    yd = _dev(np.full(B * ho * wo * c8 + 16, 0x1234, np.uint16))
+    ops.dwconv(d, xd.data_ptr(), packed.data_ptr(), rd.data_ptr() if res else None, yd.data_ptr(), B)
+    y = _host(yd)
+    assert np.all(y[-16:] == 0x1234) and np.all(y[:-16].reshape(-1, c8)[:, c:] == 0x1234)
+    got = _from_nhwc(y[:-16], B, c, ho, wo)
+    for b in (0, B - 1):
+        ref = O.conv2d(x[b * c * h * w:(b + 1) * c * h * w], wt, bias,
+                       None if r is None else r[b * c * ho * wo:(b + 1) * c * ho * wo],
+                       c, h, w, c, k, s, p, c, ho, wo, act, O.F32, 2)
+        assert _ok(got[b], ref, f"depthwise {c} k{k} s{s} image {b}")
