@@ -232,7 +232,7 @@ bool conv1x1_nchw8_ok(const ConvParams & p)
 }
 
 // Row-tiled stem for the common case (kernels/conv_cin3.cl:67-118 semantics): 3x3 stride 2
-// pad 1, Cin <= 3, Cout <= 16, planar NCHW input, channels-last output, no residual.  A
+// pad 1, Cin <= 3, Cout <= 16, planar NCHW input, no residual (channels-last output first).  A
 // work-group owns TR output rows of one image.  It stages the 2*TR+1 input rows it needs in
 // LDS as [row][col][4] (channels interleaved, 4th slot zero; two zero columns on each side
 // for the padding), loading each channel plane with 16-byte coalesced loads.  Each wave then
@@ -240,16 +240,21 @@ bool conv1x1_nchw8_ok(const ConvParams & p)
 // tap 8), B fragments are two 8-byte LDS reads per lane, weights ([16][64], k = tap*4 + ci)
 // stay in registers, and the D layout gives each lane 4 consecutive channels of one pixel,
 // so a block is 16 pixels x 32 bytes written contiguously.
-template <int TR, int UIT, int ACT>
+// VW: pixels per staged piece (8, or 4 for widths that are no multiple of 8).  PL: planar
+// output.  The MFMA operands change places, so a lane holds four consecutive pixels of one
+// channel, written as 8 bytes of that plane (16 channels, 640x640, batch 64: 318 us on the
+// conv_stem_mfma_kernel -> 107 us).
+template <int TR, int UIT, int ACT, int VW = 8, bool PL = false>
 __global__ void __launch_bounds__(256) conv_stem_rows_kernel(const ConvParams p)
 {
+  typedef _Float16 hw_t __attribute__((ext_vector_type(VW)));
   extern __shared__ __attribute__((aligned(16))) _Float16 srow[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // XCD-aware order over (row tile, image): consecutive row tiles share an input row
   const int lin = xcd_tile(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x * gridDim.y);
   const int b = lin / gridDim.x, oy0 = (lin % gridDim.x) * TR;
   const int W = p.W, LW = W + 4;               // LDS row: 2 pad columns each side
-  const int G = W >> 3;                        // 8-pixel column groups per input row
+  const int G = W / VW;                        // VW-pixel column groups per input row
   const float inv_g = __builtin_amdgcn_rcpf((float)G);
   const _Float16 * xb = reinterpret_cast<const _Float16 *>(p.x.ptr) + (long)b * p.x.img;
   // zero the pad columns of every staged row
@@ -259,26 +264,26 @@ __global__ void __launch_bounds__(256) conv_stem_rows_kernel(const ConvParams p)
     *reinterpret_cast<h4s *>(srow + ((long)lr * LW + col) * 4) = h4s{};
   }
   // every load of this thread is issued before the first LDS store (UIT units of three
-  // 16-byte channel loads; the host keeps (2*TR+1)*W/8 <= 256*UIT)
-  h8s c[UIT][3];
+  // channel loads; the host keeps (2*TR+1)*W/VW <= 256*UIT)
+  hw_t c[UIT][3];
   int dsto[UIT];
 #pragma unroll
   for (int i = 0; i < UIT; ++i) {
     const int u = tid + 256 * i;
     const int lr = idiv_small(u, G, inv_g), g = u - lr * G;
     const int iy = 2 * oy0 - 1 + lr;
-    dsto[i] = u < (2 * TR + 1) * G ? (lr * LW + 8 * g + 2) * 4 : -1;
+    dsto[i] = u < (2 * TR + 1) * G ? (lr * LW + VW * g + 2) * 4 : -1;
     const bool ok = dsto[i] >= 0 && iy >= 0 && iy < p.H;
 #pragma unroll
     for (int ci = 0; ci < 3; ++ci)
-      c[i][ci] = (ok && ci < p.Cin) ? *reinterpret_cast<const h8s *>(xb + (long)ci * p.x.cs + (long)iy * W + 8 * g) : h8s{};
+      c[i][ci] = (ok && ci < p.Cin) ? *reinterpret_cast<const hw_t *>(xb + (long)ci * p.x.cs + (long)iy * W + VW * g) : hw_t{};
   }
 #pragma unroll
   for (int i = 0; i < UIT; ++i) {
     if (dsto[i] < 0) continue;
     _Float16 * dst = srow + dsto[i];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < VW / 2; ++j) {
       h8s v;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
@@ -301,14 +306,19 @@ __global__ void __launch_bounds__(256) conv_stem_rows_kernel(const ConvParams p)
   const h8s a2 = *reinterpret_cast<const h8s *>(W4 + co * 64 + 32 + 8 * q);
   float bias[4];
 #pragma unroll
-  for (int v = 0; v < 4; ++v) bias[v] = (p.bias && 4 * q + v < p.Cout) ? p.bias[4 * q + v] : 0.0f;
+  for (int v = 0; v < 4; ++v) {
+    const int cv = PL ? co : 4 * q + v;  // the channel of the lane's accumulator v
+    bias[v] = (p.bias && cv < p.Cout) ? p.bias[cv] : 0.0f;
+  }
   // LDS offsets (halves) of the lane's taps relative to its pixel's window corner
   const int ta = 2 * q, tb = 2 * q + 1;
   const int off0 = ((ta / 3) * LW + ta % 3) * 4, off1 = ((tb / 3) * LW + tb % 3) * 4;
   const int off8 = (2 * LW + 2) * 4;
   const int CB = (p.Wo + 15) >> 4;
   const int px = lane & 15;
-  _Float16 * const yb = reinterpret_cast<_Float16 *>(p.y.ptr) + (long)b * p.y.img + 4 * q;
+  _Float16 * const yb = reinterpret_cast<_Float16 *>(p.y.ptr) + (long)b * p.y.img + (PL ? (long)co * p.y.cs : 4 * q);
+  // PL: rows of whole 4-pixel runs at 8-byte boundaries
+  const bool run4 = PL && ((p.Wo | p.y.cs | (int)(p.y.img & 3) | (int)(reinterpret_cast<uintptr_t>(p.y.ptr) >> 1)) & 3) == 0;
   const bool full = 4 * q + 4 <= p.Cout;
   // blocks (output row r, 16-pixel column block cb); wave w takes cb = w, w + 4, ... four
   // blocks per pass: all LDS fragment reads first, then the MFMAs and the stores
@@ -316,7 +326,7 @@ __global__ void __launch_bounds__(256) conv_stem_rows_kernel(const ConvParams p)
     const int oy = oy0 + r;
     if (oy >= p.Ho) break;
     const _Float16 * const rbase = srow + (2 * r * LW + 1) * 4;
-    _Float16 * const yrow = yb + (long)oy * p.Wo * p.y.cs;
+    _Float16 * const yrow = yb + (long)oy * p.Wo * (PL ? 1 : p.y.cs);
     for (int cb0 = wave; cb0 < CB; cb0 += 16) {
       h8s b1[4], b2[4];
 #pragma unroll
@@ -338,6 +348,23 @@ __global__ void __launch_bounds__(256) conv_stem_rows_kernel(const ConvParams p)
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         f4s acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        if constexpr (PL) {
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(b1[k], a1, acc, 0, 0, 0);
+          acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(b2[k], a2, acc, 0, 0, 0);
+          const int ox = (cb0 + 4 * k) * 16 + 4 * q;  // first of the lane's four pixels
+          if (cb0 + 4 * k >= CB || ox >= p.Wo || co >= p.Cout) continue;
+          h4s hv;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) hv[v] = (_Float16)act_fast<ACT>(acc[v] + bias[v]);
+          if (run4) {
+            *reinterpret_cast<h4s *>(yrow + ox) = hv;
+          } else {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+              if (ox + v < p.Wo) yrow[ox + v] = hv[v];
+          }
+          continue;
+        }
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, b1[k], acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a2, b2[k], acc, 0, 0, 0);
         const int ox = (cb0 + 4 * k) * 16 + px;
@@ -364,16 +391,26 @@ static long stem_rows_lds(int W) { return (long)(2 * kStemTR + 1) * (W + 4) * 8;
 bool stem_rows_supported(const ConvParams & p)
 {
   auto al = [](const void * ptr, int bytes) { return (reinterpret_cast<uintptr_t>(ptr) % bytes) == 0; };
+  const bool y_ok = p.y.layout == kNCHW || ((p.y.cs % 4) == 0 && (p.y.img % 4) == 0 && al(p.y.ptr, 8) && p.W % 8 == 0);
+  const int vw = p.W % 8 ? 4 : 8;  // pixels per staged piece; 4 only with planar output
   return p.stem_mfma && p.w2 && p.K == 3 && p.S == 2 && p.P == 1 && p.G == 1 && p.Cin >= 1 && p.Cin <= 3 &&
-         p.Cout <= 16 && !p.r.ptr && p.x.layout == kNCHW && p.y.layout == kNHWC && (p.W % 8) == 0 &&
-         (p.x.cs % 8) == 0 && (p.x.img % 8) == 0 && al(p.x.ptr, 16) && (p.y.cs % 4) == 0 && (p.y.img % 4) == 0 &&
-         al(p.y.ptr, 8) && p.Ho == (p.H - 1) / 2 + 1 && p.Wo == (p.W - 1) / 2 + 1 && stem_rows_lds(p.W) <= 65536 &&
-         (2 * kStemTR + 1) * (p.W / 8) <= 256 * kStemUIT;
+         p.Cout <= 16 && !p.r.ptr && p.x.layout == kNCHW && y_ok && (p.W % vw) == 0 && (p.x.cs % vw) == 0 &&
+         (p.x.img % vw) == 0 && al(p.x.ptr, 2 * vw) && p.Ho == (p.H - 1) / 2 + 1 && p.Wo == (p.W - 1) / 2 + 1 &&
+         stem_rows_lds(p.W) <= 65536 && (2 * kStemTR + 1) * (p.W / vw) <= 256 * kStemUIT * (8 / vw);
 }
 
 bool stem_supported(const ConvParams & p)
 {
   return p.K == 3 && p.G == 1 && p.Cin >= 1 && p.Cin <= 3 && p.Cout <= 32 && p.stem_mfma;
+}
+
+template <int ACT>
+static void launch_stem_rows(const ConvParams & p, dim3 grid, size_t lds, hipStream_t s)
+{
+  constexpr int TR = kStemTR, UIT = kStemUIT;
+  if (p.y.layout != kNCHW) hipLaunchKernelGGL((conv_stem_rows_kernel<TR, UIT, ACT>), grid, dim3(256), lds, s, p);
+  else if (p.W % 8 == 0) hipLaunchKernelGGL((conv_stem_rows_kernel<TR, UIT, ACT, 8, true>), grid, dim3(256), lds, s, p);
+  else hipLaunchKernelGGL((conv_stem_rows_kernel<TR, 2 * UIT, ACT, 4, true>), grid, dim3(256), lds, s, p);
 }
 
 void launch_conv_direct(const ConvParams & p, hipStream_t s)
@@ -382,12 +419,12 @@ void launch_conv_direct(const ConvParams & p, hipStream_t s)
     const dim3 grid((unsigned)((p.Ho + kStemTR - 1) / kStemTR), (unsigned)p.batch);
     const size_t lds = (size_t)stem_rows_lds(p.W);
     switch (p.act) {
-    case kActSiLU: hipLaunchKernelGGL((conv_stem_rows_kernel<kStemTR, kStemUIT, kActSiLU>), grid, dim3(256), lds, s, p); break;
-    case kActReLU: hipLaunchKernelGGL((conv_stem_rows_kernel<kStemTR, kStemUIT, kActReLU>), grid, dim3(256), lds, s, p); break;
-    case kActHSwish: hipLaunchKernelGGL((conv_stem_rows_kernel<kStemTR, kStemUIT, kActHSwish>), grid, dim3(256), lds, s, p); break;
-    case kActHSigmoid: hipLaunchKernelGGL((conv_stem_rows_kernel<kStemTR, kStemUIT, kActHSigmoid>), grid, dim3(256), lds, s, p); break;
-    case kActSigmoid: hipLaunchKernelGGL((conv_stem_rows_kernel<kStemTR, kStemUIT, kActSigmoid>), grid, dim3(256), lds, s, p); break;
-    default: hipLaunchKernelGGL((conv_stem_rows_kernel<kStemTR, kStemUIT, kActNone>), grid, dim3(256), lds, s, p); break;
+    case kActSiLU: launch_stem_rows<kActSiLU>(p, grid, lds, s); break;
+    case kActReLU: launch_stem_rows<kActReLU>(p, grid, lds, s); break;
+    case kActHSwish: launch_stem_rows<kActHSwish>(p, grid, lds, s); break;
+    case kActHSigmoid: launch_stem_rows<kActHSigmoid>(p, grid, lds, s); break;
+    case kActSigmoid: launch_stem_rows<kActSigmoid>(p, grid, lds, s); break;
+    default: launch_stem_rows<kActNone>(p, grid, lds, s); break;
     }
     return;
   }

@@ -405,3 +405,33 @@ def test_abi_depthwise_ragged_channels(c, h, w, k, s, B, res):
                        None if r is None else r[b * c * ho * wo:(b + 1) * c * ho * wo],
                        c, h, w, c, k, s, p, c, ho, wo, act, O.F32, 2)
         assert _ok(got[b], ref, f"depthwise {c} k{k} s{s} image {b}")
+
+
+@pytest.mark.parametrize("cin,cout,h,w,B,act", [
+    (3, 16, 64, 64, 2, ops.ACT_SILU),    # whole 16-pixel blocks, 8-byte stores
+    (3, 16, 28, 28, 3, ops.ACT_HSWISH),  # width a multiple of 4: 8-byte pieces, rows of 14 outputs
+    (3, 9, 33, 40, 1, ops.ACT_RELU),     # odd height, ragged channels
+    (2, 16, 6, 12, 2, ops.ACT_NONE),     # fewer pixels than a block, rows of 6
+    (1, 1, 5, 4, 1, ops.ACT_SILU),
+    (3, 16, 8, 816, 1, ops.ACT_SILU),    # the widest staged rows of 4-pixel pieces
+    (3, 16, 8, 820, 1, ops.ACT_SILU),    # ... and wider: the general kernel
+])
+def test_abi_stem_planes(cin, cout, h, w, B, act):
+    """The 3x3 stride-2 stem from planes to planes."""
+    rng = np.random.default_rng(w)
+    d = ops.conv_desc(cin, cout, h, w, 3, 2, 1, act=act, channels_last=False)
+    ho, wo = ops.conv_out_dims(d)
+    x = O.f2h((rng.random(B * cin * h * w) * 2 - 1).astype(np.float32))
+    wt = O.f2h((rng.standard_normal(cout * cin * 9) * np.sqrt(2.0 / (cin * 9))).astype(np.float32))
+    bias = O.f2h((rng.standard_normal(cout) * 0.1).astype(np.float32))
+    packed = _pack(d, wt, bias)
+    n = B * cout * ho * wo
+    xd, yd = _dev(x), _dev(np.full(n + 16, NAN16, np.uint16))
+    ops.conv2d(d, xd.data_ptr(), packed.data_ptr(), None, yd.data_ptr(), B)
+    y = _host(yd)
+    assert np.all(y[n:] == NAN16)
+    got = y[:n].reshape(B, -1)
+    for b in range(B):
+        ref = O.conv2d(x[b * cin * h * w:(b + 1) * cin * h * w], wt, bias, None, cin, h, w, cout, 3, 2, 1, 1, ho, wo,
+                       act, O.F32, 0)
+        assert _ok(got[b], ref, f"stem {cin}->{cout} {h}x{w} image {b}")
