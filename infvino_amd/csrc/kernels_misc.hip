@@ -510,9 +510,11 @@ constexpr int kDwMaxW = 4;  // weight pieces per lane: K*K*G <= 1024
 
 // Eight channels of a pixel, or the first n of a last piece past which the channels belong to no
 // output of this conv.  (Its inputs there, padding that may hold anything, reach only them.)
+// RAG: the channel count is no multiple of 8 (compile-time, the test costs the others 1 %).
+template <bool RAG>
 __device__ __forceinline__ void dw_store(_Float16 * y, const h8 & v, int n)
 {
-  if (n >= 8) {
+  if (!RAG || n >= 8) {
     *reinterpret_cast<h8 *>(y) = v;
   } else {
 #pragma unroll
@@ -521,7 +523,7 @@ __device__ __forceinline__ void dw_store(_Float16 * y, const h8 & v, int n)
   }
 }
 
-template <int K, int S, int PX, int PY, int ACT>
+template <int K, int S, int PX, int PY, int ACT, bool RAG>
 __global__ void __launch_bounds__(256) dw_tile_kernel(const ConvParams p, const DwTile t)
 {
   extern __shared__ __align__(16) unsigned char dw_lds[];
@@ -539,10 +541,10 @@ __global__ void __launch_bounds__(256) dw_tile_kernel(const ConvParams p, const 
   const int ix0 = ox0 * S - p.P, iy0 = oy0 * S - p.P, c0 = tc * G * 8;
 
   // this image's input view from channel c0 on, up to its last pixel's last 8-channel piece
-  const int C8 = (p.Cin + 7) >> 3;
+  const int C8 = RAG ? (p.Cin + 7) >> 3 : p.Cin >> 3;
   const __half * xb = p.x.ptr + (long)b * p.x.img + c0;
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<__half *>(xb), (short)0, (int)((((long)p.H * p.W - 1) * p.x.cs + C8 * 8 - c0) * 2), kBufDword3);
+      const_cast<__half *>(xb), (short)0, (int)((((long)p.H * p.W - 1) * p.x.cs + (RAG ? C8 * 8 : p.Cin) - c0) * 2), kBufDword3);
   const h8 * wg = reinterpret_cast<const h8 *>(p.w2) + tc * G;
   h8 * const xs = reinterpret_cast<h8 *>(dw_lds);  // [IH][IW][G] window pieces, then [K*K][G] weights
   // window piece i = tid + 256 u: row i / RP of the window, piece rem = i % RP of that row
@@ -656,7 +658,7 @@ __global__ void __launch_bounds__(256) dw_tile_kernel(const ConvParams p, const 
 #pragma unroll
         for (int e = 0; e < 8; ++e) out[e] = (_Float16)((float)out[e] + (float)rv[e]);
       }
-      dw_store(yb + hw * p.y.cs, out, p.Cin - c);
+      dw_store<RAG>(yb + hw * p.y.cs, out, p.Cin - c);
     }
   }
 }
@@ -667,13 +669,13 @@ __global__ void __launch_bounds__(256) dw_tile_kernel(const ConvParams p, const 
 // kernel's window is about 4x its output tile and every tap is an LDS read; measured on
 // MI355X (72 channels, 28x28 -> 14x14, batch 256) this kernel takes 11.7 us against the
 // tiled kernel's 15.5, while at batch 64 the tiled kernel wins (6.7 against 7.5 us).
-template <int K, int S, int PX, int ACT>
+template <int K, int S, int PX, int ACT, bool RAG>
 __global__ void __launch_bounds__(256) dw_strip_kernel(const ConvParams p, FastDiv d_c8, FastDiv d_strip, FastDiv d_ho)
 {
   // lane = (8-channel group, strip of PX output pixels of one row), channel groups fastest so
   // that neighbouring lanes read and write neighbouring 16-byte pieces
   constexpr int NX = (PX - 1) * S + K;  // input columns of a strip
-  const int C8 = (p.Cin + 7) >> 3, nstrip = (p.Wo + PX - 1) / PX;
+  const int C8 = RAG ? (p.Cin + 7) >> 3 : p.Cin >> 3, nstrip = (p.Wo + PX - 1) / PX;
   const unsigned idx = blockIdx.x * 256u + threadIdx.x;
   const unsigned q = fastdiv(idx, d_c8), rowi = fastdiv(q, d_strip), b = fastdiv(rowi, d_ho);
   if (b >= (unsigned)p.batch) return;
@@ -699,7 +701,7 @@ __global__ void __launch_bounds__(256) dw_strip_kernel(const ConvParams p, FastD
     }
 #pragma unroll
     for (int kx = 0; kx < K; ++kx) {
-      const h8 wv = *reinterpret_cast<const h8 *>(W + (ky * K + kx) * (C8 * 8));
+      const h8 wv = *reinterpret_cast<const h8 *>(W + (ky * K + kx) * (RAG ? C8 * 8 : p.Cin));
 #pragma unroll
       for (int j = 0; j < PX; ++j) {
         const h8 v = xv[j * S + kx];
@@ -729,7 +731,7 @@ __global__ void __launch_bounds__(256) dw_strip_kernel(const ConvParams p, FastD
 #pragma unroll
       for (int e = 0; e < 8; ++e) out[e] = (_Float16)((float)out[e] + (float)rv[e]);
     }
-    dw_store(yb + hw * p.y.cs, out, p.Cin - c);
+    dw_store<RAG>(yb + hw * p.y.cs, out, p.Cin - c);
   }
 }
 
@@ -917,21 +919,28 @@ static DwPick dw_pick(const ConvParams & p)
   return d;
 }
 
-template <int K, int S, int PX, int PY>
-static void launch_dw_tile(const ConvParams & p, const DwPick & d, hipStream_t s)
+template <int K, int S, int PX, int PY, bool RAG>
+static void launch_dw_tile_r(const ConvParams & p, const DwPick & d, hipStream_t s)
 {
   const unsigned nwg = (unsigned)((long)d.t.ntx * d.t.nty * d.t.nct * p.batch);
   switch (p.act) {
 #define IVH_DW_CASE(A)                                                                                     \
-  case A: hipLaunchKernelGGL((dw_tile_kernel<K, S, PX, PY, A>), dim3(nwg), dim3(256), d.lds, s, p, d.t); break;
+  case A: hipLaunchKernelGGL((dw_tile_kernel<K, S, PX, PY, A, RAG>), dim3(nwg), dim3(256), d.lds, s, p, d.t); break;
   IVH_DW_CASE(kActSiLU)
   IVH_DW_CASE(kActReLU)
   IVH_DW_CASE(kActHSwish)
   IVH_DW_CASE(kActHSigmoid)
   IVH_DW_CASE(kActSigmoid)
-  default: hipLaunchKernelGGL((dw_tile_kernel<K, S, PX, PY, kActNone>), dim3(nwg), dim3(256), d.lds, s, p, d.t); break;
+  default: hipLaunchKernelGGL((dw_tile_kernel<K, S, PX, PY, kActNone, RAG>), dim3(nwg), dim3(256), d.lds, s, p, d.t); break;
 #undef IVH_DW_CASE
   }
+}
+
+template <int K, int S, int PX, int PY>
+static void launch_dw_tile(const ConvParams & p, const DwPick & d, hipStream_t s)
+{
+  if (p.Cin % 8) launch_dw_tile_r<K, S, PX, PY, true>(p, d, s);
+  else launch_dw_tile_r<K, S, PX, PY, false>(p, d, s);
 }
 
 template <int K, int S>
@@ -949,8 +958,10 @@ static void launch_dw_strip(const ConvParams & p, hipStream_t s)
   const int nstrip = (p.Wo + PX - 1) / PX;
   const int C8 = (p.Cin + 7) / 8;
   const long n = (long)p.batch * p.Ho * nstrip * C8;
-  hipLaunchKernelGGL((dw_strip_kernel<5, 2, PX, ACT>), dim3(nblk(n, 256)), dim3(256), 0, s, p,
-                     fastdiv_make((unsigned)C8), fastdiv_make((unsigned)nstrip), fastdiv_make((unsigned)p.Ho));
+  const dim3 g(nblk(n, 256));
+  const FastDiv f8 = fastdiv_make((unsigned)C8), fs = fastdiv_make((unsigned)nstrip), fh = fastdiv_make((unsigned)p.Ho);
+  if (p.Cin % 8) hipLaunchKernelGGL((dw_strip_kernel<5, 2, PX, ACT, true>), g, dim3(256), 0, s, p, f8, fs, fh);
+  else hipLaunchKernelGGL((dw_strip_kernel<5, 2, PX, ACT, false>), g, dim3(256), 0, s, p, f8, fs, fh);
 }
 
 // The strip kernel is taken for 5x5 stride 2 once it has at least 1.5 waves per SIMD.
