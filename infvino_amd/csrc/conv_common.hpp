@@ -89,6 +89,15 @@ __device__ __forceinline__ float act_fast(float v)
   return v;
 }
 
+// One fp32 -> fp16 rounding of a finished value.  The empty asm keeps the compiler from fusing
+// the value's last multiply with the conversion in some copies of an epilogue and not in
+// others (one rounding instead of two): an output must not depend on which copy made it.
+__device__ __forceinline__ _Float16 round_f16(float v)
+{
+  __asm__("" : "+v"(v));
+  return (_Float16)v;
+}
+
 // MFMA block of MB x MB outputs.  Operand A = weights (row i = output channel), operand B =
 // pixels (column j = pixel); each lane supplies 8 consecutive K values of one row / column.
 //   MB = 32: v_mfma_f32_32x32x16_f16, K slice 16, lane k offset 8*(lane/32);

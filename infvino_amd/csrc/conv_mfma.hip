@@ -461,7 +461,7 @@ std::string igemm_launch_tag(const ConvParams & p)
     snprintf(b, sizeof b, "cfg=%d th=%d tw=%d", p.s2 - 1, p.th, p.tw);
   else
     snprintf(b, sizeof b, "bn=%d bk=%d ksplit=%d%s%s%s%s%s", igemm_bn(p.Cout), p.ring ? 32 : p.bk, p.ksplit,
-             p.ring == 2 ? " dma k-halves" : p.ring ? " dma" : "", !p.ring && igemm_occ4(p) ? " vgpr128" : "", p.xt ? " planar" : "", (p.Cin & 7) ? " cin-ragged" : "",
+             p.ring == 3 ? " streamed" : p.ring == 2 ? " dma k-halves" : p.ring ? " dma" : "", !p.ring && igemm_occ4(p) ? " vgpr128" : "", p.xt ? " planar" : "", (p.Cin & 7) ? " cin-ragged" : "",
              p.cu ? " upsample-concat" : "");
   return b;
 }
@@ -499,6 +499,10 @@ void launch_conv_igemm(const ConvParams & p, hipStream_t s)
   }
   if (p.s2) {
     launch_conv_s2(p, s);
+    return;
+  }
+  if (p.ring == 3) {
+    launch_conv_stream(p, s);
     return;
   }
   if (p.ring) {

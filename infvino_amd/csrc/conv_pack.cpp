@@ -81,10 +81,11 @@ bool use_small(const ConvSpec & s, ConvParams & p)
   return true;
 }
 
-// the DMA-fed build of the implicit GEMM where it is the faster one
+// the streaming 1x1 kernel or the DMA-fed build of the implicit GEMM where faster (same sums but
+// for the build with K halves)
 void use_ring(const ConvSpec & s, ConvParams & p)
 {
-  p.ring = ring_plan(p, (s.flags & IVH_FLAG_NO_SPLITK) != 0);
+  p.ring = stream_plan(p) ? 3 : ring_plan(p, (s.flags & IVH_FLAG_NO_SPLITK) != 0);
   if (!p.ring) return;
   p.ksplit = 1;
   p.ws = nullptr;

@@ -68,7 +68,7 @@ __device__ __forceinline__ void ring_epilogue(const ConvParams & p, Mf<32>::acc_
           const float bb[4] = {b4.x, b4.y, b4.z, b4.w};
           h4 hv;
 #pragma unroll
-          for (int k = 0; k < 4; ++k) hv[k] = (_Float16)act_fast<ACT>(acc[tn][tm][v4 + k] + bb[k]);
+          for (int k = 0; k < 4; ++k) hv[k] = round_f16(act_fast<ACT>(acc[tn][tm][v4 + k] + bb[k]));
           h[s] = __builtin_bit_cast(u2, hv);
         }
         const auto s0 = __builtin_amdgcn_permlane32_swap(h[0][0], h[1][0], false, false);

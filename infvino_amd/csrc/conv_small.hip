@@ -281,7 +281,7 @@ __global__ void __launch_bounds__(64 * NW) conv_small_kernel(const ConvParams p)
       case kActSigmoid: v = act_fast<kActSigmoid>(v); break;
       default: break;
       }
-      hv[k] = (_Float16)v;
+      hv[k] = round_f16(v);
     }
     if (rbase) {
 #pragma unroll

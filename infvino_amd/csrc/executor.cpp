@@ -2311,7 +2311,8 @@ void Model::validate(const Launch & l) const
           throw std::runtime_error("small-grid conv geometry");
         check(p.w, 0, (long)(p.Cout + 63) / 64 * 64 * p.kpad - 1, 2, "small-grid conv w");
       }
-      if (p.ring && (p.ring > 2 || p.small || p.halo || p.res || p.pipe || p.wide || p.s2 || p.pw || p.ksplit != 1 || !ring_ok(p)))
+      if (p.ring && (p.ring > 3 || p.small || p.halo || p.res || p.pipe || p.wide || p.s2 || p.pw || p.ksplit != 1 ||
+                     !(p.ring == 3 ? stream_ok(p) : ring_ok(p))))
         throw std::runtime_error("DMA-fed implicit-GEMM geometry");
       if (p.halo) {
         const int cfg = p.halo - 1, ck = p.ck;

@@ -98,7 +98,8 @@ struct ConvParams {
   // small-grid implicit GEMM (conv_small.hip, K split over a work-group's waves): config + 1
   // (0: not used); w is the implicit-GEMM packing
   int small = 0;
-  // implicit GEMM fed by LDS DMA (conv_ring.hip): 1, or 2 with the K range in halves; 0: not used
+  // implicit GEMM fed by LDS DMA (conv_ring.hip): 1, or 2 with the K range in halves;
+  // 3: the streaming 1x1 kernel (conv_stream.hip); 0: not used
   int ring = 0;
   // implicit GEMM of a 1x1 conv reading NCHW channel planes (x.cs = pixels per plane, a
   // multiple of 8): each thread loads 8 consecutive pixels of one channel and writes them

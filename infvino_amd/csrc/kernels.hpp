@@ -38,6 +38,11 @@ bool ring_ok(const ConvParams & p);
 int ring_plan(const ConvParams & p, bool one_order);  // 0: conv_igemm_kernel, 1: whole K, 2: K halves
 void launch_conv_ring(const ConvParams & p, hipStream_t s);
 
+// conv_stream.hip: 1x1 convs with 64 < Cout <= 128, weights in registers, pixels streamed
+bool stream_ok(const ConvParams & p);
+bool stream_plan(const ConvParams & p);  // ... and it is the faster one
+void launch_conv_stream(const ConvParams & p, hipStream_t s);
+
 // conv_halo.hip: 3x3 stride-1 pad-1 convs with an LDS input patch
 constexpr int kHaloCfgs = 9;         // tile configs of the LDS-patch kernel
 int halo_cfg_ck(int cfg, int cin);  // input-channel chunk a tile config uses (16 / 32 / 64)

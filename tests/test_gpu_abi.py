@@ -344,6 +344,9 @@ def test_abi_softmax_rows(axis):
     (264, 40, 33, 35, 1, 1, 20, True),    # the same, 9 steps, 40 of 64 channels
     (40, 256, 53, 53, 1, 1, 7, False),    # whole K: two steps, the second ragged
     (32, 136, 61, 59, 3, 2, 40, True),    # whole K with taps, a second channel tile of 8
+    (192, 128, 64, 64, 1, 1, 16, False),  # streamed pixels: four blocks a work-group
+    (136, 72, 81, 83, 1, 1, 11, False),   # a chunk of 8 channels, 8 of a wave's channels, a last block of 17 pixels
+    (384, 104, 90, 91, 1, 1, 13, False),  # six chunks, uneven shares
 ])
 def test_abi_dma_implicit_gemm(cin, cout, h, w, k, s, B, res):
     """Implicit-GEMM convs through the DMA-fed kernel: image 0 and the last one against the oracle,
