@@ -839,6 +839,12 @@ bool dwconv_vectorizable(const ConvParams & p)
 // 2.5 waves per SIMD hide their load latency; below that the candidate with the most waves
 // is taken (small batches); among those with enough, work-groups of two or more waves, then
 // the cheapest.
+// Where none of these fits, any block of at most 256 lanes is a candidate (147 channels on
+// 160-pixel rows: 19 groups in sixteenths of a row, ten columns, exceed the window), and then any
+// divisor of the groups (325 channels are 41 groups, a prime, whose 5x5 weights exceed the
+// staging registers): one group and one pixel always fit.  147 channels 3x3 at 160x160, batch 4:
+// 34.5 us (540 us on the any-layout kernel; 42.7 us with one group a tile); 325 channels 5x5 at
+// 20x20, batch 16: 12.2 us (229 us).
 struct DwPick {
   int PX = 0, PY = 0;
   DwTile t{};
@@ -853,11 +859,41 @@ static DwPick dw_pick_search(const ConvParams & p)
   DwPick best;
   double best_cost = 1e300, best_wk = 0.0;
   bool best_big = false;
+  auto consider = [&](int PX, int PY, int G, int BX, int BY) {
+    const int NR = (PY - 1) * S + K, NX = (PX - 1) * S + K;
+    const int lanes = G * BX * BY;
+    if (lanes > 256) return;
+    const int IW = (BX * PX - 1) * S + K, IH = (BY * PY - 1) * S + K;
+    const int nbuf = (IH * IW + K * K) * G;
+    if (nbuf > kDwBufPieces || K * K * G > kDwMaxW * 256) return;
+    const int ntx = (p.Wo + BX * PX - 1) / (BX * PX), nty = (p.Ho + BY * PY - 1) / (BY * PY);
+    const double nwg = (double)ntx * nty * (C8 / G) * p.batch;
+    if (nwg >= 2147483648.0) return;
+    const double waves = nwg * ((lanes + 63) / 64);
+    const double valu = waves * (PX * PY * K * K * 8 + ((nbuf + 255) / 256) * 25 + 150) * 4.0 / 1024.0;
+    const double lds = nwg * (nbuf + (double)lanes * (NR * NX + K * K)) * 16.0 / (256.0 * 128.0);
+    const double mem = hbm / 2500.0 + nwg * IH * IW * G * 16.0 / 10000.0;
+    const double cost = std::max(valu, std::max(lds, mem));
+    // rank: waves up to enough; then work-groups of at least two waves (one-wave
+    // groups pay the staging latency for a quarter of the lanes); then cost
+    const double wk = std::min(waves, kEnoughWaves);
+    const bool big = lanes >= 128;
+    const bool better = best.PX == 0 || wk > best_wk || (wk == best_wk && big > best_big) ||
+                        (wk == best_wk && big == best_big && cost < best_cost);
+    if (better) {
+      best_cost = cost;
+      best_wk = wk;
+      best_big = big;
+      best.PX = PX;
+      best.PY = PY;
+      best.t = DwTile{G, BX, BY, ntx, nty, C8 / G, IW, IH};
+      best.lds = (size_t)nbuf * 16;
+    }
+  };
   for (const int PX : {1, 2}) {
     for (const int PY : {1, 2}) {
       if (PX * PY > 2) continue;
       const int nbx = (p.Wo + PX - 1) / PX, nby = (p.Ho + PY - 1) / PY;
-      const int NR = (PY - 1) * S + K, NX = (PX - 1) * S + K;
       for (int G = 1; G <= C8; ++G) {
         if (C8 % G || (G < C8 && G < 8)) continue;
         for (int sx = 1, last_bx = 0; sx <= nbx && sx <= 16; ++sx) {
@@ -868,37 +904,18 @@ static DwPick dw_pick_search(const ConvParams & p)
             const int BY = (nby + sy - 1) / sy;
             if (BY == last_by) continue;
             last_by = BY;
-            const int lanes = G * BX * BY;
-            if (lanes > 256) continue;
-            const int IW = (BX * PX - 1) * S + K, IH = (BY * PY - 1) * S + K;
-            const int nbuf = (IH * IW + K * K) * G;
-            if (nbuf > kDwBufPieces || K * K * G > kDwMaxW * 256) continue;
-            const int ntx = (p.Wo + BX * PX - 1) / (BX * PX), nty = (p.Ho + BY * PY - 1) / (BY * PY);
-            const double nwg = (double)ntx * nty * (C8 / G) * p.batch;
-            if (nwg >= 2147483648.0) continue;
-            const double waves = nwg * ((lanes + 63) / 64);
-            const double valu = waves * (PX * PY * K * K * 8 + ((nbuf + 255) / 256) * 25 + 150) * 4.0 / 1024.0;
-            const double lds = nwg * (nbuf + (double)lanes * (NR * NX + K * K)) * 16.0 / (256.0 * 128.0);
-            const double mem = hbm / 2500.0 + nwg * IH * IW * G * 16.0 / 10000.0;
-            const double cost = std::max(valu, std::max(lds, mem));
-            // rank: waves up to enough; then work-groups of at least two waves (one-wave
-            // groups pay the staging latency for a quarter of the lanes); then cost
-            const double wk = std::min(waves, kEnoughWaves);
-            const bool big = lanes >= 128;
-            const bool better = best.PX == 0 || wk > best_wk || (wk == best_wk && big > best_big) ||
-                                (wk == best_wk && big == best_big && cost < best_cost);
-            if (better) {
-              best_cost = cost;
-              best_wk = wk;
-              best_big = big;
-              best.PX = PX;
-              best.PY = PY;
-              best.t = DwTile{G, BX, BY, ntx, nty, C8 / G, IW, IH};
-              best.lds = (size_t)nbuf * 16;
-            }
+            consider(PX, PY, G, BX, BY);
           }
         }
       }
+    }
+  }
+  for (const int g_min : {8, 1}) {
+    if (best.PX) break;
+    for (int G = 1; G <= C8 && G <= 256; ++G) {
+      if (C8 % G || (G < C8 && G < g_min)) continue;
+      for (int BX = 1; BX <= p.Wo && G * BX <= 256; ++BX)
+        for (int BY = 1; BY <= p.Ho && G * BX * BY <= 256; ++BY) consider(1, 1, G, BX, BY);
     }
   }
   return best;

@@ -383,6 +383,9 @@ def test_abi_dma_implicit_gemm(cin, cout, h, w, k, s, B, res):
 @pytest.mark.parametrize("c,h,w,k,s,B,res", [
     (2, 5, 5, 3, 1, 2, False), (7, 9, 11, 5, 2, 1, True), (9, 14, 14, 3, 2, 3, False), (51, 20, 20, 3, 1, 4, True),
     (145, 13, 17, 5, 1, 2, False), (70, 28, 28, 5, 2, 256, False), (33, 112, 112, 3, 1, 2, False),
+    (325, 20, 20, 5, 1, 2, True),    # 41 groups, a prime: tiles of one group
+    (328, 13, 9, 5, 1, 3, False),    # the same without a partial group
+    (147, 160, 160, 3, 1, 1, True),  # 19 groups on rows of 160 pixels: two columns a tile
 ])
 def test_abi_depthwise_ragged_channels(c, h, w, k, s, B, res):
     """Depthwise convs whose channel count leaves a partial last piece (tile and strip kernels):

@@ -201,6 +201,34 @@ def test_launch_tags(tmp_path, shape, head, detail, flags):
     assert tag.startswith(head) and detail in tag.split(), tag
 
 
+def test_depthwise_tile_for_every_channel_count(tmp_path):
+    """The depthwise planner finds a tile within the kernel's limits (256 lanes, 4096 LDS pieces,
+    1024 weight pieces) for every channel count, those whose groups of 8 have no divisor that
+    the usual tiles take among them (41, 43, 47 groups 5x5; 19 groups on 160-pixel rows)."""
+    for c8 in range(1, 73):
+        for h, w in ((7, 7), (20, 20), (53, 160), (160, 160)):
+            c = 8 * c8 - (5 if (c8 + h) % 2 else 0)
+            pb = pw.PlanBuilder(str(tmp_path), 0)
+            x = pb.unary(pb.input("x", [1, c, h, w]), pw.UN_RELU)
+            geo = [(3, 1), (3, 2), (5, 1), (5, 2)]
+            for k, s in geo:
+                pb.output(pb.unary(pb.conv(x, c, k, s, groups=c, act=pw.ACT_SILU), pw.UN_RELU))
+            m = ia.PlanModel(pb.write(), 0, 1, DRY)
+            m.run(1)
+            tags = [m.nodeTag(i) for i in range(m.nodeCount()) if m.nodeInfo(i)["kernel"] == "dwconv"]
+            m.close()
+            assert len(tags) == 4
+            for (k, s), tag in zip(geo, tags):
+                if tag.split()[1] != "tile":
+                    continue  # another kernel, which has no tile to find
+                t = dict(f.split("=") for f in tag.split()[2:])
+                px, py, g, bx, by = (int(t[f]) for f in ("px", "py", "g", "bx", "by"))
+                label = f"{c} channels {h}x{w} k{k} s{s}: {tag}"
+                assert min(px, py, g, bx, by) >= 1 and c8 % g == 0 and g * bx * by <= 256, label
+                window = ((bx * px - 1) * s + k) * ((by * py - 1) * s + k)
+                assert (window + k * k) * g <= 4096 and k * k * g <= 1024, label
+
+
 def test_zero_copy_views_in_c2f(plans):
     """C2f: cv1 output is split by views, the bottleneck outputs and both halves land in the
     concat buffer in place, so no copy_c/concat node launches anything."""
