@@ -554,7 +554,7 @@ __global__ void __launch_bounds__(256) dw_tile_kernel(const ConvParams p, const 
   const int jlo = max(0, -ix0) * G, jhi = (p.W - ix0) * G;  // a row's pieces inside the image
   // byte offsets: window origin (may be negative; only in-image pieces use it), one image row,
   // one pixel; 24-bit multiplies (full rate) suffice, the host keeps an image below 2^31 bytes
-  // and its pixel count below 2^24
+  // and a row below 2^24 (dw_kind)
   const int base0 = (iy0 * p.W + ix0) * p.x.cs * 2, rowb = p.W * p.x.cs * 2, pixb = p.x.cs * 2;
   h8 v[kDwMaxIt];
   auto load_window = [&](auto contig) {
@@ -987,11 +987,29 @@ static bool dw_use_strip(const ConvParams & p)
   return p.K == 5 && p.S == 2 && (long)p.batch * p.Ho * ((p.Wo + 3) / 4) * ((p.Cin + 7) / 8) >= 1536L * 64;
 }
 
+enum class DwKind { kStrip, kTile, kPlanar, kAny };
+
+// The kernel of a depthwise conv.  The tiled kernel multiplies row numbers by an image row's
+// bytes in 24 bits: longer rows run on the any-layout kernel.
+static DwKind dw_kind(const ConvParams & p)
+{
+  if (dwconv_vectorizable(p)) {
+    if (dw_use_strip(p)) return DwKind::kStrip;
+    return (long)p.W * p.x.cs * 2 < (1L << 24) ? DwKind::kTile : DwKind::kAny;
+  }
+  const bool planar = p.x.layout == kNCHW && (long)p.H * p.W < (1L << 31) && (p.K == 3 || p.K == 5) &&
+                      (p.S == 1 || p.S == 2);
+  return planar ? DwKind::kPlanar : DwKind::kAny;
+}
+
 std::string dw_launch_tag(const ConvParams & p)
 {
-  if (!dwconv_vectorizable(p))
-    return p.x.layout == kNCHW && (p.K == 3 || p.K == 5) && (p.S == 1 || p.S == 2) ? "planar px=4" : "generic";
-  if (dw_use_strip(p)) return "strip px=4";
+  switch (dw_kind(p)) {
+  case DwKind::kStrip: return "strip px=4";
+  case DwKind::kPlanar: return "planar px=4";
+  case DwKind::kAny: return "generic";
+  case DwKind::kTile: break;
+  }
   const DwPick d = dw_pick(p);
   char b[128];
   snprintf(b, sizeof b, "tile px=%d py=%d g=%d bx=%d by=%d", d.PX, d.PY, d.t.G, d.t.BX, d.t.BY);
@@ -1000,12 +1018,10 @@ std::string dw_launch_tag(const ConvParams & p)
 
 void launch_dwconv(const ConvParams & p, hipStream_t s)
 {
-  if (!dwconv_vectorizable(p)) {
+  const DwKind kind = dw_kind(p);
+  if (kind == DwKind::kPlanar || kind == DwKind::kAny) {
     if (p.Cin > 65535 || p.batch > 65535) throw std::runtime_error("depthwise: grid");
-    const dim3 grid(nblk((long)p.Ho * p.Wo, 256), (unsigned)p.Cin, (unsigned)p.batch);
-    const bool planar = p.x.layout == kNCHW && (long)p.H * p.W < (1L << 31) && (p.K == 3 || p.K == 5) &&
-                        (p.S == 1 || p.S == 2);
-    if (planar) {
+    if (kind == DwKind::kPlanar) {
       constexpr int PX = 4;
       const int strips = (p.Wo + PX - 1) / PX;
       const long n = (long)p.Cin * p.Ho * strips;
@@ -1017,11 +1033,12 @@ void launch_dwconv(const ConvParams & p, hipStream_t s)
       else if (p.S == 1) hipLaunchKernelGGL((dw_nchw_kernel<5, 1, PX>), g, dim3(256), 0, s, p, f, fp);
       else hipLaunchKernelGGL((dw_nchw_kernel<5, 2, PX>), g, dim3(256), 0, s, p, f, fp);
     } else {
+      const dim3 grid(nblk((long)p.Ho * p.Wo, 256), (unsigned)p.Cin, (unsigned)p.batch);
       hipLaunchKernelGGL(dw_generic_kernel, grid, dim3(256), 0, s, p, fastdiv_make((unsigned)p.Wo));
     }
     return;
   }
-  if (dw_use_strip(p)) {
+  if (kind == DwKind::kStrip) {
     switch (p.act) {
     case kActSiLU: launch_dw_strip<kActSiLU>(p, s); break;
     case kActReLU: launch_dw_strip<kActReLU>(p, s); break;

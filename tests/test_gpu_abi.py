@@ -386,6 +386,7 @@ def test_abi_dma_implicit_gemm(cin, cout, h, w, k, s, B, res):
     (325, 20, 20, 5, 1, 2, True),    # 41 groups, a prime: tiles of one group
     (328, 13, 9, 5, 1, 3, False),    # the same without a partial group
     (147, 160, 160, 3, 1, 1, True),  # 19 groups on rows of 160 pixels: two columns a tile
+    (65, 3, 116600, 3, 1, 1, False),  # rows of more than 2^24 bytes: the any-layout kernel
 ])
 def test_abi_depthwise_ragged_channels(c, h, w, k, s, B, res):
     """Depthwise convs whose channel count leaves a partial last piece (tile and strip kernels):

@@ -229,6 +229,18 @@ def test_depthwise_tile_for_every_channel_count(tmp_path):
                 assert (window + k * k) * g <= 4096 and k * k * g <= 1024, label
 
 
+@pytest.mark.parametrize("w,want", [(116400, "tile"), (116600, "generic")])
+def test_depthwise_long_rows(tmp_path, w, want):
+    """The tiled depthwise kernel's 24-bit row offsets hold up to rows of 2^24 bytes (72 channels
+    a pixel); longer rows run on the any-layout kernel."""
+    path, _ = pw.single_conv(str(tmp_path), 65, 65, 3, w, k=3, groups=65, act=pw.ACT_SILU, pre_relu=True, post_relu=True)
+    m = ia.PlanModel(path, 0, 1, DRY)
+    m.run(1)
+    tag = next(m.nodeTag(i) for i in range(m.nodeCount()) if m.nodeInfo(i)["kernel"] == "dwconv")
+    m.close()
+    assert tag.split()[1] == want, tag
+
+
 def test_zero_copy_views_in_c2f(plans):
     """C2f: cv1 output is split by views, the bottleneck outputs and both halves land in the
     concat buffer in place, so no copy_c/concat node launches anything."""
