@@ -507,6 +507,7 @@ __device__ __forceinline__ void fma_mix(float & acc, unsigned a, unsigned b)
 constexpr int kDwMaxIt = 16;
 constexpr int kDwBufPieces = kDwMaxIt * 256;
 constexpr int kDwMaxW = 4;  // weight pieces per lane: K*K*G <= 1024
+constexpr double kDwMaxWgs = 16777216.0;  // a launch holds fewer than 2^32 lanes per grid dimension
 
 // Eight channels of a pixel, or the first n of a last piece past which the channels belong to no
 // output of this conv.  (Its inputs there, padding that may hold anything, reach only them.)
@@ -842,7 +843,8 @@ bool dwconv_vectorizable(const ConvParams & p)
 // Where none of these fits, any block of at most 256 lanes is a candidate (147 channels on
 // 160-pixel rows: 19 groups in sixteenths of a row, ten columns, exceed the window), and then any
 // divisor of the groups (325 channels are 41 groups, a prime, whose 5x5 weights exceed the
-// staging registers): one group and one pixel always fit.  147 channels 3x3 at 160x160, batch 4:
+// staging registers): one group and one pixel always fit, unless
+// that is too many work-groups for a launch (dw_kind).  147 channels 3x3 at 160x160, batch 4:
 // 34.5 us (540 us on the any-layout kernel; 42.7 us with one group a tile); 325 channels 5x5 at
 // 20x20, batch 16: 12.2 us (229 us).
 struct DwPick {
@@ -868,7 +870,7 @@ static DwPick dw_pick_search(const ConvParams & p)
     if (nbuf > kDwBufPieces || K * K * G > kDwMaxW * 256) return;
     const int ntx = (p.Wo + BX * PX - 1) / (BX * PX), nty = (p.Ho + BY * PY - 1) / (BY * PY);
     const double nwg = (double)ntx * nty * (C8 / G) * p.batch;
-    if (nwg >= 2147483648.0) return;
+    if (nwg >= kDwMaxWgs) return;
     const double waves = nwg * ((lanes + 63) / 64);
     const double valu = waves * (PX * PY * K * K * 8 + ((nbuf + 255) / 256) * 25 + 150) * 4.0 / 1024.0;
     const double lds = nwg * (nbuf + (double)lanes * (NR * NX + K * K)) * 16.0 / (256.0 * 128.0);
@@ -989,13 +991,17 @@ static bool dw_use_strip(const ConvParams & p)
 
 enum class DwKind { kStrip, kTile, kPlanar, kAny };
 
-// The kernel of a depthwise conv.  The tiled kernel multiplies row numbers by an image row's
-// bytes in 24 bits: longer rows run on the any-layout kernel.
-static DwKind dw_kind(const ConvParams & p)
+// The kernel of a depthwise conv, with the pick for the tiled one.  That kernel multiplies row
+// numbers by an image row's bytes in 24 bits: longer rows run on the any-layout kernel, and so
+// do convs of more tiles than a launch holds (2051 channels, whose 257 groups are a prime, of
+// 65535 images).
+static DwKind dw_kind(const ConvParams & p, DwPick & d)
 {
   if (dwconv_vectorizable(p)) {
     if (dw_use_strip(p)) return DwKind::kStrip;
-    return (long)p.W * p.x.cs * 2 < (1L << 24) ? DwKind::kTile : DwKind::kAny;
+    if ((long)p.W * p.x.cs * 2 >= (1L << 24)) return DwKind::kAny;
+    d = dw_pick(p);
+    return d.PX ? DwKind::kTile : DwKind::kAny;
   }
   const bool planar = p.x.layout == kNCHW && (long)p.H * p.W < (1L << 31) && (p.K == 3 || p.K == 5) &&
                       (p.S == 1 || p.S == 2);
@@ -1004,13 +1010,13 @@ static DwKind dw_kind(const ConvParams & p)
 
 std::string dw_launch_tag(const ConvParams & p)
 {
-  switch (dw_kind(p)) {
+  DwPick d;
+  switch (dw_kind(p, d)) {
   case DwKind::kStrip: return "strip px=4";
   case DwKind::kPlanar: return "planar px=4";
   case DwKind::kAny: return "generic";
   case DwKind::kTile: break;
   }
-  const DwPick d = dw_pick(p);
   char b[128];
   snprintf(b, sizeof b, "tile px=%d py=%d g=%d bx=%d by=%d", d.PX, d.PY, d.t.G, d.t.BX, d.t.BY);
   return b;
@@ -1018,7 +1024,8 @@ std::string dw_launch_tag(const ConvParams & p)
 
 void launch_dwconv(const ConvParams & p, hipStream_t s)
 {
-  const DwKind kind = dw_kind(p);
+  DwPick d;
+  const DwKind kind = dw_kind(p, d);
   if (kind == DwKind::kPlanar || kind == DwKind::kAny) {
     if (p.Cin > 65535 || p.batch > 65535) throw std::runtime_error("depthwise: grid");
     if (kind == DwKind::kPlanar) {
@@ -1049,8 +1056,6 @@ void launch_dwconv(const ConvParams & p, hipStream_t s)
     }
     return;
   }
-  const DwPick d = dw_pick(p);
-  if (d.PX == 0) throw std::runtime_error("depthwise: no tile fits");
   if (p.K == 3) {
     if (p.S == 1) launch_dw_ks<3, 1>(p, d, s);
     else launch_dw_ks<3, 2>(p, d, s);

@@ -233,11 +233,23 @@ def test_depthwise_tile_for_every_channel_count(tmp_path):
 def test_depthwise_long_rows(tmp_path, w, want):
     """The tiled depthwise kernel's 24-bit row offsets hold up to rows of 2^24 bytes (72 channels
     a pixel); longer rows run on the any-layout kernel."""
-    path, _ = pw.single_conv(str(tmp_path), 65, 65, 3, w, k=3, groups=65, act=pw.ACT_SILU, pre_relu=True, post_relu=True)
-    m = ia.PlanModel(path, 0, 1, DRY)
-    m.run(1)
+    assert _dw_tag(tmp_path, 65, 3, w, 3, 1).split()[1] == want
+
+
+def _dw_tag(tmp_path, c, h, w, k, batch):
+    path, _ = pw.single_conv(str(tmp_path), c, c, h, w, k=k, groups=c, act=pw.ACT_SILU, pre_relu=True, post_relu=True)
+    m = ia.PlanModel(path, 0, batch, DRY)
+    m.run(batch)
     tag = next(m.nodeTag(i) for i in range(m.nodeCount()) if m.nodeInfo(i)["kernel"] == "dwconv")
     m.close()
+    return tag
+
+
+@pytest.mark.parametrize("c,batch,want", [(2051, 65000, "tile"), (2051, 65500, "generic"), (2043, 65500, "tile")])
+def test_depthwise_work_group_limit(tmp_path, c, batch, want):
+    """A launch holds fewer than 2^24 work-groups of 256 lanes; 257 one-group tiles of more than
+    65280 images run on the any-layout kernel instead."""
+    tag = _dw_tag(tmp_path, c, 7, 7, 3, batch)
     assert tag.split()[1] == want, tag
 
 
