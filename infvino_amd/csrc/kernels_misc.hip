@@ -994,14 +994,28 @@ enum class DwKind { kStrip, kTile, kPlanar, kAny };
 // The kernel of a depthwise conv, with the pick for the tiled one.  That kernel multiplies row
 // numbers by an image row's bytes in 24 bits: longer rows run on the any-layout kernel, and so
 // do convs of more tiles than a launch holds (2051 channels, whose 257 groups are a prime, of
-// 65535 images).
+// 65535 images).  A partial last group (Cin % 8) with little work in many work-groups stays there
+// as well: the tiled kernel's time then is that of its work-groups (about 3.6 us + 2.2 us per
+// thousand of up to 63 lanes), the any-layout kernel's that of its taps (2.6 us + 1.1 / 1.6 /
+// 3.0 us per million at up to 7 / 23 / more channels, at least 4.2 us 3x3 and 6.2 us 5x5: one
+// lane per value, whose taps are a pixel apart).  Measured on 300 shapes of 2-576 channels, 5-160
+// pixels a side, 1-256 images: 7 channels 3x3 at 7x7, batch 64: 4.2 against 10.0 us; 33 at 20x20,
+// batch 8: 5.8 against 6.8; 33 at 40x40, batch 8: 14.4 against 8.4 us.
 static DwKind dw_kind(const ConvParams & p, DwPick & d)
 {
   if (dwconv_vectorizable(p)) {
     if (dw_use_strip(p)) return DwKind::kStrip;
     if ((long)p.W * p.x.cs * 2 >= (1L << 24)) return DwKind::kAny;
     d = dw_pick(p);
-    return d.PX ? DwKind::kTile : DwKind::kAny;
+    if (!d.PX) return DwKind::kAny;
+    const int C = p.Cin, lanes = d.t.G * d.t.BX * d.t.BY;
+    if (C % 8 && lanes < 64) {
+      const double wgs = (double)d.t.ntx * d.t.nty * d.t.nct * p.batch;
+      const double macs = (double)p.batch * p.Ho * p.Wo * C * p.K * p.K;
+      const double any = 2.6 + macs * (C < 8 ? 1.1e-6 : C < 24 ? 1.6e-6 : 3.0e-6);
+      if (std::max(any, p.K == 3 ? 4.2 : 6.2) < 3.6 + wgs * 2.2e-3) return DwKind::kAny;
+    }
+    return DwKind::kTile;
   }
   const bool planar = p.x.layout == kNCHW && (long)p.H * p.W < (1L << 31) && (p.K == 3 || p.K == 5) &&
                       (p.S == 1 || p.S == 2);

@@ -236,13 +236,29 @@ def test_depthwise_long_rows(tmp_path, w, want):
     assert _dw_tag(tmp_path, 65, 3, w, 3, 1).split()[1] == want
 
 
-def _dw_tag(tmp_path, c, h, w, k, batch):
-    path, _ = pw.single_conv(str(tmp_path), c, c, h, w, k=k, groups=c, act=pw.ACT_SILU, pre_relu=True, post_relu=True)
+def _dw_tag(tmp_path, c, h, w, k, batch, s=1):
+    path, _ = pw.single_conv(str(tmp_path), c, c, h, w, k=k, s=s, groups=c, act=pw.ACT_SILU, pre_relu=True,
+                             post_relu=True)
     m = ia.PlanModel(path, 0, batch, DRY)
     m.run(batch)
     tag = next(m.nodeTag(i) for i in range(m.nodeCount()) if m.nodeInfo(i)["kernel"] == "dwconv")
     m.close()
     return tag
+
+
+@pytest.mark.parametrize("c,h,w,k,s,batch,want", [
+    # the GPU tests' shapes
+    (9, 14, 14, 3, 2, 3, "tile"), (145, 13, 17, 5, 1, 2, "tile"), (33, 112, 112, 3, 1, 2, "tile"),
+    (147, 160, 160, 3, 1, 1, "tile"), (70, 28, 28, 5, 2, 256, "strip"), (51, 20, 20, 3, 1, 4, "generic"),
+    # measured: tens of thousands of values in thousands of small tiles, and more of them
+    (7, 7, 7, 3, 1, 64, "generic"), (33, 20, 20, 3, 1, 8, "generic"), (15, 7, 7, 5, 2, 256, "generic"),
+    (33, 40, 40, 3, 1, 8, "tile"), (25, 20, 20, 3, 1, 64, "tile"), (15, 160, 160, 5, 2, 1, "tile"),
+    (16, 7, 7, 3, 1, 64, "tile"),  # whole groups of 8: always the tiled kernel
+])
+def test_depthwise_partial_group_kernel(tmp_path, c, h, w, k, s, batch, want):
+    """Which kernel a channel count that is no multiple of 8 runs on."""
+    tag = _dw_tag(tmp_path, c, h, w, k, batch, s)
+    assert tag.split()[1] == want, tag
 
 
 @pytest.mark.parametrize("c,batch,want", [(2051, 65000, "tile"), (2051, 65500, "generic"), (2043, 65500, "tile")])
