@@ -77,7 +77,7 @@ ivh::ConvSpec conv_spec(const ivh_conv_desc * d, bool gemv)
   // 1x1 on planes of whole 8-pixel pieces, as the plan executor routes them: the MFMA kernels
   // (64->128 at 80x80, one image: 35.7 us a call on the direct kernel, 5.2 us).  Up to 8 output channels
   // the direct family's vector kernel, which is no slower, stays; so do odd planes and, from
-  // the same blob, pointers off a 16-byte boundary.
+  // the same blob, pointers off a 16-byte boundary and a few input channels (conv_resolve).
   s.x_planes8 = s.keep_direct = !s.x_nhwc && !gemv && s.G == 1 && s.K == 1 && s.S == 1 && s.P == 0 && s.Cout > 8 &&
                                 (long)s.H * s.W % 8 == 0 && (long)s.H * s.W < (1L << 27);
   if (s.Ho() < 1 || s.Wo() < 1) throw std::invalid_argument("conv descriptor: empty output");

@@ -66,6 +66,19 @@ bool planes_vec_ok(const ConvParams & p)
   return true;
 }
 
+// 1x1 convs on planes of so few input channels that the direct kernel, whose time is about
+// Cin's, stays ahead.  Against the implicit GEMM's 128-channel tiles on few pixels: 1->200 at
+// 20x20 6.6 vs 9.0 us, 2->200 at 80x80 7.5 vs 8.1, 4->128 at 20x20 8.2 vs 8.8 (5->200 at 80x80 8.8
+// vs 8.1, 3->200 at 20x20, batch 64: 11.6 vs 10.9).  Against either MFMA kernel with few outputs
+// of many pixels, where both are bound by memory: 1->9 at 320x320, batch 4 / 16: 10.8 vs 13.2
+// us, 1.47 times; 2->16, batch 16: 1.11 times; 3->16 the same, 5->9 0.95 times; 1->32 0.72 times.
+bool planes_direct_faster(const ConvParams & p)
+{
+  const long px = (long)p.batch * p.H * p.W;
+  if (p.Cout <= 16 && p.Cin * p.Cout < 56 && px >= 100000) return true;
+  return p.Cin <= 5 && p.Cout > 64 && p.Cin * px < (p.Cin == 1 ? 30000 : 14000) && !pwt_plan(p);
+}
+
 // the small-grid kernel where it is the faster one; not with NO_SPLITK, under which an image's
 // fp32 sums have one order at every batch size
 bool use_small(const ConvSpec & s, ConvParams & p)
@@ -231,12 +244,12 @@ int conv_resolve(const ConvSpec & s, const ConvPacking & pk, const void * dev_bl
     if (pk.stem && pk.stem_w2 != kNoSeg) p.w2 = reinterpret_cast<const __half *>(base + pk.stem_w2);
     return kLaunchDirect;
   }
-  if (pk.direct != kNoSeg && !planes_vec_ok(p)) {
+  p.cin8 = pk.cin8;
+  p.kpad = pk.kpad;
+  if (pk.direct != kNoSeg && (!planes_vec_ok(p) || planes_direct_faster(p))) {
     p.w = reinterpret_cast<const __half *>(base + pk.direct);
     return kLaunchDirect;
   }
-  p.cin8 = pk.cin8;
-  p.kpad = pk.kpad;
   p.bk = igemm_bk(p.Cout, p.K * p.K * p.cin8);
   p.ksplit = 1;
   p.ws = nullptr;

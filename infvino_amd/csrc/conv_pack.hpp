@@ -26,8 +26,8 @@ struct ConvSpec {
   bool x_vec1 = false;  // single-pixel NCHW input (an FC / GEMV): the MFMA family reads it too
   bool x_planes8 = false;  // 1x1 conv on NCHW input whose planes hold a multiple of 8 pixels:
                            // the MFMA family reads it, transposing pixel pieces in LDS
-  bool keep_direct = false;  // x_planes8 and the caller's pointers may lack 16-byte alignment:
-                             // the blob also holds the direct kernel's weights
+  bool keep_direct = false;  // x_planes8, and the batch or the caller's pointers may ask for the
+                             // direct kernel: the blob also holds its weights
   bool lone = false;    // a single-op call, not a plan's node
   uint32_t flags = 0;   // IVH_FLAG_DIRECT_ONLY / IVH_FLAG_NO_HALO
   int Ho() const { return (H + 2 * P - K) / S + 1; }

@@ -235,6 +235,9 @@ def test_abi_maxpool_planes(k, c, h, w, batch, off):
     (24, 33, 6, 20, True, 1),     # pointers one element off a 16-byte boundary: the direct kernel
     (24, 8, 6, 20, False, 0),     # up to 8 output channels, and ...
     (24, 33, 5, 5, False, 0),     # ... planes of an odd size: the direct family
+    (2, 130, 8, 8, True, 0),      # a few input channels: the direct kernel, here on few pixels, ...
+    (3, 9, 192, 200, False, 0),   # ... here with few outputs of many
+    (3, 40, 8, 8, False, 0),      # few input channels on the planar streaming kernel
 ])
 def test_abi_pointwise_planes(cin, cout, h, w, res, off):
     B, n_in, n_out = 3, cin * h * w, cout * h * w
