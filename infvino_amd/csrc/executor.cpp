@@ -2716,8 +2716,10 @@ bool Model::ringReady()
 // Measured into a fresh array: 60 MB of fp16 5.3 ms by the runtime's copy, 4.8 / 3.0 / 1.9 /
 // 1.6 ms with 1 / 2 / 4 / 8 threads; 120 MB as f32 40 ms (converted on the host) -> 2.9 ms;
 // one image's head as f32 (1.9 MB) 392 -> 75 us (95 us in chunks of 1 MB).
-void Model::ringRead(char * dst, size_t bytes, const std::function<void(char *, size_t, size_t)> & fill)
+bool Model::ringRead(char * dst, size_t bytes, const std::function<void(char *, size_t, size_t)> & fill)
 {
+  std::lock_guard<std::mutex> lock(ring_mu_);
+  if (!ringReady()) return false;
   const size_t ch = bytes < ((size_t)8 << 20) ? kRingChunk / 2 : kRingChunk;
   const long nc = (long)((bytes + ch - 1) / ch);
   const int cpus = std::max(1, (int)std::thread::hardware_concurrency() / 2);
@@ -2763,6 +2765,7 @@ void Model::ringRead(char * dst, size_t bytes, const std::function<void(char *, 
       (void)hipStreamSynchronize(stream_);  // nothing of this call may still write the ring
       std::rethrow_exception(e);
     }
+  return true;
 }
 
 void Model::readOutputF16(int i, uint16_t * host, int batch)
@@ -2776,13 +2779,13 @@ void Model::readOutputF16(int i, uint16_t * host, int batch)
   // large reads of images stored back to back: through the pinned ring (from 2 MB; the runtime's
   // own copy takes the same 54 us for 0.9 MB, and 380 against 273 us for 7.5 MB)
   const size_t bytes = (size_t)t.numel * 2 * batch;
-  if ((batch == 1 || v.img == t.numel) && bytes >= ((size_t)2 << 20) && !dry_ && ringReady()) {
+  if ((batch == 1 || v.img == t.numel) && bytes >= ((size_t)2 << 20) && !dry_) {
     const char * src = reinterpret_cast<const char *>(v.ptr);
-    ringRead(reinterpret_cast<char *>(host), bytes, [&](char * pin, size_t off, size_t len) {
+    auto fill = [&](char * pin, size_t off, size_t len) {
       launch_copy_out(src + off, pin, (long)len, stream_);
       HIPCHECK(hipGetLastError());
-    });
-    return;
+    };
+    if (ringRead(reinterpret_cast<char *>(host), bytes, fill)) return;
   }
   HIPCHECK(hipMemcpy2DAsync(host, t.numel * 2, v.ptr, v.img * 2, t.numel * 2, batch, hipMemcpyDeviceToHost, stream_));
   HIPCHECK(hipStreamSynchronize(stream_));
@@ -2796,12 +2799,12 @@ void Model::readOutputF32(int i, float * host, int batch)
   HIPCHECK(hipSetDevice(device_));
   const View v = view(t.name, batch);
   // the device converts, writing the floats straight into the pinned ring
-  if (!dry_ && v.layout == kNCHW && (batch == 1 || v.img == t.numel) && ringReady()) {
-    ringRead(reinterpret_cast<char *>(host), (size_t)t.numel * 4 * batch, [&](char * pin, size_t off, size_t len) {
+  if (!dry_ && v.layout == kNCHW && (batch == 1 || v.img == t.numel)) {
+    auto fill = [&](char * pin, size_t off, size_t len) {
       launch_f16_to_f32(v.ptr + off / 4, reinterpret_cast<float *>(pin), (long)(len / 4), stream_);
       HIPCHECK(hipGetLastError());
-    });
-    return;
+    };
+    if (ringRead(reinterpret_cast<char *>(host), (size_t)t.numel * 4 * batch, fill)) return;
   }
   const long n = (long)outputNumel(i);
   std::vector<uint16_t> h((size_t)n * batch);

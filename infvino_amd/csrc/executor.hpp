@@ -8,6 +8,7 @@
 #include <functional>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -172,11 +173,13 @@ class Model {
   // read that needs it and given back with the model
   static constexpr int kRingSlots = 16, kRingThreads = 8;
   static constexpr size_t kRingChunk = 1 << 20;
+  std::mutex ring_mu_;  // held by a read that uses the ring: two threads may read one model's outputs
   char * ring_ = nullptr;
   hipEvent_t ring_ev_[kRingSlots] = {};
   bool ringReady();
-  // `dst[0, bytes)` from chunks that fill(pinned chunk, offset, bytes) enqueues on the stream
-  void ringRead(char * dst, size_t bytes, const std::function<void(char *, size_t, size_t)> & fill);
+  // `dst[0, bytes)` from chunks that fill(pinned chunk, offset, bytes) enqueues on the stream;
+  // false, with nothing done, without pinned memory
+  bool ringRead(char * dst, size_t bytes, const std::function<void(char *, size_t, size_t)> & fill);
   void * stage_f32_ = nullptr;              // f32 staging for the truncating conversion
   std::vector<void *> dev_allocs_;          // weights etc.
   size_t weight_bytes_ = 0;

@@ -373,3 +373,36 @@ def test_readback_sizes(tmp_path, hw, batch):
         f = m.readOutputF32(0, batch)
         assert np.array_equal(f.view(np.uint32), O.h2f(x).view(np.uint32))
     m.close()
+
+
+def test_readback_from_two_threads(tmp_path):
+    """Two threads reading outputs of one model at once: each read is whole (they share the
+    model's pinned ring)."""
+    import threading
+    hw, batch = 1024, 4
+    n = hw * hw
+    path = tmp_path / "two.plan"
+    path.write_text(f"input x 1 1 {hw} {hw}\ntensor y 1 1 {hw} {hw}\ntensor z 1 1 {hw} {hw}\n"
+                    f"node copy_c x y HW={n} c0=0 cnt=1 dst_off=0\nnode ew_unary x z op=2 n={n}\noutput y\noutput z\n")
+    m = ia.PlanModel(str(path), 0, batch, ia.IVH_FLAG_NO_FUSE)
+    x = O.f2h((np.arange(n * batch) % 4001 - 2000).astype(np.float32))
+    m.setInput(x, batch)
+    m.run(batch)
+    want = [m.readOutput(i, batch) for i in (0, 1)]
+    assert np.array_equal(want[0], x) and np.array_equal(O.h2f(want[1]), np.maximum(O.h2f(x), 0))
+    bad = []
+
+    def read(i):
+        for _ in range(20):
+            if not np.array_equal(m.readOutput(i, batch), want[i]):
+                bad.append(("f16", i))
+            if not np.array_equal(m.readOutputF32(i, batch), O.h2f(want[i])):
+                bad.append(("f32", i))
+
+    threads = [threading.Thread(target=read, args=(i,)) for i in (0, 1)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    m.close()
+    assert not bad, bad
