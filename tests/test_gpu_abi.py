@@ -4,10 +4,13 @@ compared with the CPU oracle on the same seeded inputs, with the op-level bar of
 tests (fp32 oracle: mean_rel < 2e-3, max_rel < 1e-2; data movement bit-exact).  The
 padding channels of channels-last activations hold NaN bit patterns, so a kernel that lets
 them reach an output fails."""
+import time
+
 import numpy as np
 import pytest
 import torch
 
+import infvino_amd as ia
 import infvino_amd.ops as ops
 from oracle import oracle as O
 
@@ -445,3 +448,29 @@ def test_abi_stem_planes(cin, cout, h, w, B, act):
         ref = O.conv2d(x[b * cin * h * w:(b + 1) * cin * h * w], wt, bias, None, cin, h, w, cout, 3, 2, 1, 1, ho, wo,
                        act, O.F32, 0)
         assert _ok(got[b], ref, f"stem {cin}->{cout} {h}x{w} image {b}")
+
+
+def test_readback_into_pinned_memory(tmp_path):
+    """A pinned destination: the same values, and, as one copy without the ring's detour, no
+    slower than the same read into pageable memory."""
+    hw, batch = 1024, 8
+    n = hw * hw
+    path = tmp_path / "io.plan"
+    path.write_text(f"input x 1 1 {hw} {hw}\ntensor y 1 1 {hw} {hw}\nnode copy_c x y HW={n} c0=0 cnt=1 dst_off=0\noutput y\n")
+    m = ia.PlanModel(str(path), 0, batch, ia.IVH_FLAG_NO_FUSE)
+    x = np.resize(np.arange(65536, dtype=np.uint16), n * batch)
+    m.setInput(x, batch)
+    m.run(batch)
+    took = []
+    for pin in (True, False):
+        buf = torch.zeros(n * batch, dtype=torch.int16, pin_memory=pin)
+        best = 1e9
+        for _ in range(6):
+            t0 = time.perf_counter()
+            assert ia.lib().ivh_read_output_f16(m._h, 0, buf.data_ptr(), batch) == 0
+            best = min(best, time.perf_counter() - t0)
+        assert np.array_equal(buf.numpy().view(np.uint16), x)
+        took.append(best)
+    print(f"16 MB: pinned {took[0] * 1e6:.0f} us, pageable {took[1] * 1e6:.0f} us")
+    m.close()
+    assert took[0] < took[1]
