@@ -2690,21 +2690,29 @@ void Model::sync()
   HIPCHECK(hipStreamSynchronize(stream_));
 }
 
-bool Model::ringReady()
+// The ring for a read of `bytes`: as large as the read, in powers of two from 64 KB, up to
+// kRingSlots chunks, so that a model of small outputs does not pin 16 MB.  (Pinned memory that is new
+// to the process costs the first copy out of it 0.37 ms per MB, mapped page by page; fewer
+// slots or smaller chunks save part of that once and cost 10-16 % of every later read.)
+bool Model::ringReady(size_t bytes)
 {
-  if (ring_) return true;
+  size_t want = (size_t)64 << 10;
+  while (want < bytes && want < kRingSlots * kRingChunk) want *= 2;
+  if (want <= ring_bytes_) return true;
+  for (auto & e : ring_ev_)
+    if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+      e = nullptr;
+      (void)hipGetLastError();
+      return false;
+    }
   void * p = nullptr;
-  if (hipHostMalloc(&p, kRingSlots * kRingChunk, hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc(&p, want, hipHostMallocDefault) != hipSuccess) {
     (void)hipGetLastError();
     return false;
   }
-  for (auto & e : ring_ev_)
-    if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-      (void)hipGetLastError();
-      (void)hipHostFree(p);
-      return false;
-    }
+  if (ring_) (void)hipHostFree(ring_);  // every read waits for its chunks: nothing is in flight
   ring_ = static_cast<char *>(p);
+  ring_bytes_ = want;
   return true;
 }
 
@@ -2719,11 +2727,12 @@ bool Model::ringReady()
 bool Model::ringRead(char * dst, size_t bytes, const std::function<void(char *, size_t, size_t)> & fill)
 {
   std::lock_guard<std::mutex> lock(ring_mu_);
-  if (!ringReady()) return false;
+  if (!ringReady(bytes)) return false;
   const size_t ch = bytes < ((size_t)8 << 20) ? kRingChunk / 2 : kRingChunk;
   const long nc = (long)((bytes + ch - 1) / ch);
   const int cpus = std::max(1, (int)std::thread::hardware_concurrency() / 2);
-  const int T = std::max(1, std::min({kRingThreads, cpus, (int)(bytes >> 22)})), S = kRingSlots / T;
+  const int T = std::max(1, std::min({kRingThreads, cpus, (int)(bytes >> 22)}));
+  const int S = std::max(1, (int)std::min<size_t>(kRingSlots, ring_bytes_ / ch) / T);
   std::exception_ptr err[kRingThreads];
   // worker t: chunks t, t + T, ... through its own S slots
   auto work = [&](int t) {
@@ -2732,7 +2741,7 @@ bool Model::ringRead(char * dst, size_t bytes, const std::function<void(char *, 
       auto issue = [&](long c) {
         const int slot = t * S + (int)(c / T % S);
         const size_t off = (size_t)c * ch, len = std::min(ch, bytes - off);
-        fill(ring_ + (size_t)slot * kRingChunk, off, len);
+        fill(ring_ + (size_t)slot * ch, off, len);
         HIPCHECK(hipEventRecord(ring_ev_[slot], stream_));
       };
       for (long c = t, k = 0; k < S && c < nc; c += T, ++k) issue(c);
@@ -2740,7 +2749,7 @@ bool Model::ringRead(char * dst, size_t bytes, const std::function<void(char *, 
         const int slot = t * S + (int)(c / T % S);
         const size_t off = (size_t)c * ch, len = std::min(ch, bytes - off);
         HIPCHECK(hipEventSynchronize(ring_ev_[slot]));
-        std::memcpy(dst + off, ring_ + (size_t)slot * kRingChunk, len);
+        std::memcpy(dst + off, ring_ + (size_t)slot * ch, len);
         if (c + (long)T * S < nc) issue(c + (long)T * S);
       }
     } catch (...) {

@@ -169,14 +169,15 @@ class Model {
   void * arena_ = nullptr;                  // activations, max_batch images
   long arena_elems1_ = 0;                   // elements per image-unit
   void * input_buf_ = nullptr;              // graph input, max_batch images (fp16)
-  // Readback through pinned host memory: a ring of kRingSlots chunks, allocated by the first
-  // read that needs it and given back with the model
+  // Readback through pinned host memory: a ring of up to kRingSlots chunks, grown by the reads
+  // that need more and given back with the model
   static constexpr int kRingSlots = 16, kRingThreads = 8;
   static constexpr size_t kRingChunk = 1 << 20;
   std::mutex ring_mu_;  // held by a read that uses the ring: two threads may read one model's outputs
   char * ring_ = nullptr;
+  size_t ring_bytes_ = 0;
   hipEvent_t ring_ev_[kRingSlots] = {};
-  bool ringReady();
+  bool ringReady(size_t bytes);
   // `dst[0, bytes)` from chunks that fill(pinned chunk, offset, bytes) enqueues on the stream;
   // false, with nothing done, without pinned memory
   bool ringRead(char * dst, size_t bytes, const std::function<void(char *, size_t, size_t)> & fill);

@@ -375,6 +375,22 @@ def test_readback_sizes(tmp_path, hw, batch):
     m.close()
 
 
+def test_readback_ring_grows(tmp_path):
+    """Reads of one image, of more chunks than the ring then holds, and of one image again."""
+    hw, batch = 300, 90
+    n = hw * hw
+    path = tmp_path / "io.plan"
+    path.write_text(f"input x 1 1 {hw} {hw}\ntensor y 1 1 {hw} {hw}\nnode copy_c x y HW={n} c0=0 cnt=1 dst_off=0\noutput y\n")
+    m = ia.PlanModel(str(path), 0, batch, ia.IVH_FLAG_NO_FUSE)
+    x = np.resize(np.arange(65536, dtype=np.uint16), n * batch)
+    m.setInput(x, batch)
+    m.run(batch)
+    for b in (1, 3, 7, 20, 50, 90, 1, 30):
+        assert np.array_equal(m.readOutputF32(0, b).view(np.uint32), O.h2f(x[:n * b]).view(np.uint32)), b
+        assert np.array_equal(m.readOutput(0, b), x[:n * b]), b
+    m.close()
+
+
 def test_readback_from_two_threads(tmp_path):
     """Two threads reading outputs of one model at once: each read is whole (they share the
     model's pinned ring)."""
