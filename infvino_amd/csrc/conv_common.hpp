@@ -91,7 +91,9 @@ __device__ __forceinline__ float act_fast(float v)
 
 // One fp32 -> fp16 rounding of a finished value.  The empty asm keeps the compiler from fusing
 // the value's last multiply with the conversion in some copies of an epilogue and not in
-// others (one rounding instead of two): an output must not depend on which copy made it.
+// others (one rounding instead of two): an output must not depend on which copy made it, nor on
+// which of the kernels with the same sums the batch size selects (implicit GEMM, its DMA-fed
+// build, the streaming 1x1 kernels).
 __device__ __forceinline__ _Float16 round_f16(float v)
 {
   __asm__("" : "+v"(v));
@@ -180,7 +182,7 @@ __device__ __forceinline__ void stage_tile(typename Mf<MB>::acc_t (&acc)[TN][TM]
         const int cl = wn * TN * MB + tn * MB + F::row(lane, v4);
         h4 hv;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) hv[k] = (_Float16)act_fast<ACT>(acc[tn][tm][v4 + k] + bv[tn][v4 + k]);
+        for (int k = 0; k < 4; ++k) hv[k] = round_f16(act_fast<ACT>(acc[tn][tm][v4 + k] + bv[tn][v4 + k]));
         if (nhwc) {
           *reinterpret_cast<h4 *>(lds + pl * (BN + 8) + cl) = hv;
         } else {

@@ -542,6 +542,40 @@ def test_split_k(tmp_path, cin, cout, hw, k, s, batch):
     assert mean_rel < 1e-3 and max_rel < 5e-3
 
 
+@pytest.mark.parametrize("cin,cout,hw,k,s,act,batch,one,many", [
+    (256, 192, 40, 1, 1, 1, 64, "dma", "conv_igemm"),
+    (128, 128, 40, 1, 1, 1, 64, "dma", "vgpr128"),
+    (384, 128, 40, 1, 1, 3, 64, "dma", "streamed"),
+    (64, 64, 80, 1, 1, 1, 64, "dma", "conv_pw"),
+    (192, 64, 80, 1, 1, 1, 64, "dma", "conv_igemm"),
+    (48, 64, 160, 1, 1, 4, 16, "dma", "conv_igemm"),
+    (32, 32, 160, 1, 1, 1, 16, "conv_igemm", "conv_pw"),
+    (256, 256, 40, 3, 2, 1, 128, "dma", "conv_igemm"),
+    (64, 256, 80, 3, 2, 5, 32, "dma", "conv_igemm"),
+])
+def test_no_splitk_bits_across_batch_sizes(tmp_path, cin, cout, hw, k, s, act, batch, one, many):
+    """With IVH_FLAG_NO_SPLITK an image of these layers has the same bits alone and in a batch
+    for which the planner picks another of the kernels that share the implicit GEMM's sums."""
+    path, _ = pw.single_conv(str(tmp_path), cin, cout, hw, hw, k=k, s=s, act=act, pre_relu=True, post_relu=True)
+    m = ia.PlanModel(path, 0, batch, ia.IVH_FLAG_NO_SPLITK)
+    n = m.inputNumel()
+    x = O.f2h((np.random.default_rng(cin).random(n * batch, dtype=np.float32) * 2 - 1))
+
+    def tag():
+        return next(m.nodeTag(i) for i in range(m.nodeCount()) if m.nodeInfo(i)["op"].startswith("conv")).split()
+
+    m.setInput(x, batch)
+    m.run(batch)
+    full = m.readOutput(0, batch).reshape(batch, -1)
+    assert many in tag() and (many == "dma" or "dma" not in tag()), tag()
+    for i in (0, batch // 2, batch - 1):
+        m.setInput(x[i * n:(i + 1) * n], 1)
+        m.run(1)
+        assert np.array_equal(m.readOutput(0, 1), full[i]), f"image {i}: {(m.readOutput(0, 1) != full[i]).sum()} values"
+    assert one in tag(), tag()
+    m.close()
+
+
 @pytest.mark.parametrize("internal,post", [(False, False), (True, False), (False, True)],
                          ids=["nchw_input", "channels_last", "nchw_in_channels_last_out"])
 @pytest.mark.parametrize("c,hw,k,s,act", [(16, 112, 3, 2, 3), (96, 14, 5, 1, 3), (72, 28, 5, 2, 3),
