@@ -105,7 +105,9 @@ __global__ void __launch_bounds__(256) conv1x1_stream_kernel(const ConvParams p)
 #pragma unroll
   for (int j = 0; j < 4; ++j) foff[j] = fbase + (((2 * j + fh) ^ fsw) * 8);
   // copies of block i are followed by those of block i + 1 and, from the second block on, by the
-  // two stores of each of the last R - 1 blocks
+  // two stores of each of the last R - 1 blocks.  The counts hold only if every block issues its
+  // copies before its stores: a store moved ahead of them would let that many copies still be in
+  // flight when their stage is read.  The empty asm after the copies pins that order.
   constexpr int W0 = NCH, W1 = NCH + 2 * (R - 1);
   auto block = [&](int i, const _Float16 * st, _Float16 * nx) __attribute__((always_inline)) {
     if (i + 1 >= n) __builtin_amdgcn_s_waitcnt(kVmWait0);
@@ -115,6 +117,7 @@ __global__ void __launch_bounds__(256) conv1x1_stream_kernel(const ConvParams p)
     __builtin_amdgcn_s_barrier();  // every wave's copies; every wave has read the stage copied next
     __asm__ volatile("" ::: "memory");
     if (i + R - 1 < n) copy(nx, i + R - 1);
+    __asm__ volatile("" ::: "memory");
     acc_t acc;
 #pragma unroll
     for (int v = 0; v < F::NV; ++v) acc[v] = 0.0f;
