@@ -22,6 +22,7 @@
 #include "conv_common.hpp"
 #include "kernels.hpp"
 
+#include <algorithm>
 #include <stdexcept>
 
 namespace ivh {
@@ -158,24 +159,63 @@ __global__ void __launch_bounds__(256) bmm_mfma_kernel(const SmallParams q, int 
   }
 }
 
+// Tile rows and columns: up to 64 columns a tile of 128 would be half empty.
+static long tiles(const SmallParams & q, long & mt, long & nt)
+{
+  const long bm = q.i3 <= 64 ? 128 : 64, bn = q.i3 <= 64 ? 64 : 128;
+  mt = (q.i1 + bm - 1) / bm;
+  nt = (q.i3 + bn - 1) / bn;
+  return mt * nt;
+}
+
 template <int TA, int TB>
 static void launch_bmm_t(const SmallParams & q, hipStream_t s)
 {
-  auto go = [&](auto BM, auto BN) {
-    constexpr int bm = decltype(BM)::value, bn = decltype(BN)::value;
-    const int mt = (q.i1 + bm - 1) / bm, nt = (q.i3 + bn - 1) / bn;
-    const long n = (long)mt * nt * q.batch * q.i0;
-    if (n >= (1L << 31) || (long)mt * nt >= (1L << 31)) throw std::runtime_error("bmm grid");
-    hipLaunchKernelGGL((bmm_mfma_kernel<TA, TB, bm, bn>), dim3((unsigned)n), dim3(256), 0, s, q, mt, nt);
-  };
-  // up to 64 columns: a tile of 128 would be half empty
-  if (q.i3 <= 64) go(std::integral_constant<int, 128>{}, std::integral_constant<int, 64>{});
-  else go(std::integral_constant<int, 64>{}, std::integral_constant<int, 128>{});
+  long mt, nt;
+  const long n = tiles(q, mt, nt) * q.batch * q.i0;
+  const dim3 grid((unsigned)n), block(256);
+  if (q.i3 <= 64) hipLaunchKernelGGL((bmm_mfma_kernel<TA, TB, 128, 64>), grid, block, 0, s, q, (int)mt, (int)nt);
+  else hipLaunchKernelGGL((bmm_mfma_kernel<TA, TB, 64, 128>), grid, block, 0, s, q, (int)mt, (int)nt);
 }
 
-// q.op bit 0: A stored [K][M]; bit 1: B stored [N][K]
+// q.op bit 0: A stored [K][M]; bit 1: B stored [N][K].  A launch holds fewer than 2^32 lanes per
+// grid dimension, 2^24 work-groups here: more tiles are launched as slices of the images, or of
+// one image's matrices.
 void launch_bmm_mfma(const SmallParams & q, hipStream_t s)
 {
+  constexpr long kMaxWgs = (1L << 24) - 1;
+  long mt, nt;
+  const long per = tiles(q, mt, nt);
+  if (per > kMaxWgs) {  // a matrix of one row or column of nearly 2^31 values (K = 1): in two parts
+    if (q.i0 != 1 || q.i2 != 1) throw std::runtime_error("bmm grid");
+    SmallParams c = q;
+    const bool rows = q.i1 > q.i3;
+    int & d = rows ? c.i1 : c.i3;
+    const int part = 1 << 30, all = d;
+    d = part;
+    launch_bmm_mfma(c, s);
+    (rows ? c.a : c.b).ptr += part;
+    c.y.ptr += part;
+    d = all - part;
+    launch_bmm_mfma(c, s);
+    return;
+  }
+  if (per * q.i0 > kMaxWgs || per * q.i0 * q.batch > kMaxWgs) {
+    const bool heads = per * q.i0 > kMaxWgs;
+    const int step = (int)(kMaxWgs / (heads ? per : per * q.i0)), all = heads ? q.i0 : q.batch;
+    for (int img = 0; img < (heads ? q.batch : 1); ++img)
+      for (int at = 0; at < all; at += step) {
+        SmallParams c = q;
+        (heads ? c.i0 : c.batch) = std::min(step, all - at);
+        if (heads) c.batch = 1;
+        const long i = heads ? img : at, h = heads ? at : 0;
+        c.a.ptr += i * q.a.img + h * q.i1 * q.i2;
+        c.b.ptr += i * q.b.img + h * q.i2 * q.i3;
+        c.y.ptr += i * q.y.img + h * q.i1 * q.i3;
+        launch_bmm_mfma(c, s);
+      }
+    return;
+  }
   switch (q.op & 3) {
   case 0: launch_bmm_t<0, 0>(q, s); break;
   case 1: launch_bmm_t<1, 0>(q, s); break;

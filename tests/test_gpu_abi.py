@@ -320,6 +320,19 @@ def test_abi_bmm_edges(bb, m, k, n, batch):
         assert _ok(got[b], ref, f"bmm {bb}x{m}x{k}x{n} image {b}")
 
 
+@pytest.mark.parametrize("bb,batch", [((1 << 18) + 1, 64), ((1 << 24) + 5, 2)])
+def test_abi_bmm_more_tiles_than_a_grid_dimension(bb, batch):
+    """2^24 and some matrices of one value: their tiles exceed one dimension of a launch, over
+    the images or within one."""
+    a = (torch.arange(bb * batch, device="cuda") % 61).half()
+    b = (torch.arange(bb * batch, device="cuda") % 29 - 14).half()
+    y = torch.full((bb * batch,), float("nan"), dtype=torch.float16, device="cuda")
+    torch.cuda.synchronize()
+    ops.bmm(a.data_ptr(), b.data_ptr(), y.data_ptr(), bb, 1, 1, 1, batch)
+    torch.cuda.synchronize()
+    assert torch.equal(y, a * b)
+
+
 @pytest.mark.parametrize("axis", [1, 7, 8, 63, 64, 65, 128, 129, 256, 399, 512, 513, 1024, 2047, 2048, 2049])
 def test_abi_softmax_rows(axis):
     """Rows of every lane count and piece count, at odd offsets, with a masked (-inf), a lowest
