@@ -1902,6 +1902,19 @@ static bool launch_maxpool_planes(const SmallParams & q, hipStream_t s)
   const long items = (long)((br + kPoolRO - 1) / kPoolRO) * ((q.W + 1) / 2);
   int G = 1;
   if (br == q.H) G = (int)std::max(1L, std::min(room / ((br + K - 1) * pd), 256 / items));
+  // a launch holds fewer than 2^32 lanes per grid dimension: more planes go in slices of the batch
+  constexpr long kMaxWgs = (1L << 24) - 1;
+  if (((long)q.batch * q.C + G - 1) / G > kMaxWgs) {
+    const int step = (int)(kMaxWgs * G / q.C);
+    for (int at = 0; at < q.batch; at += step) {
+      SmallParams c = q;
+      c.batch = std::min(step, q.batch - at);
+      c.a.ptr += (long)at * q.a.img;
+      c.y.ptr += (long)at * q.y.img;
+      if (!launch_maxpool_planes(c, s)) throw std::runtime_error("maxpool slice");
+    }
+    return true;
+  }
   const dim3 grid((unsigned)(((long)q.batch * q.C + G - 1) / G), (unsigned)((q.H + br - 1) / br));
   const size_t lds = (size_t)G * (br + K - 1) * pd * 4;
   // dword rows: even W on dense planes at a 4-byte boundary

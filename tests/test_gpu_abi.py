@@ -203,7 +203,9 @@ def test_abi_pool_softmax_bmm():
     (5, 6, 9, 10, 2, 1),       # even width at an odd element offset
     (3, 5, 4, 6, 2, 0),        # three-wide windows, one register block of rows
     (3, 2, 5, 3, 1, 0),
-    (5, 2, 200, 160, 1, 0),    # three bands of rows per plane
+    (5, 2, 200, 160, 1, 0),    # two bands of rows per plane
+    (5, 2, 300, 160, 1, 0),    # three: a band with halo rows on both sides
+    (3, 3, 331, 158, 2, 0),    # the same three rows wide, the last band shorter
     (5, 1, 9, 4001, 1, 0),     # rows so wide that a band is one register block
     (3, 1, 6, 9000, 1, 0),     # wider than a band: the scalar kernel
 ])
@@ -229,6 +231,27 @@ def test_abi_maxpool_planes(k, c, h, w, batch, off):
     y = yd.cpu().numpy()
     assert np.array_equal(y[off:off + x.size].reshape(x.shape), ref)
     assert np.all(y[:off] == 7.0) and np.all(y[off + x.size:] == 7.0)
+
+
+def test_abi_maxpool_more_planes_than_a_grid_dimension():
+    """2^24 and some planes, one to a work-group (17 GB in and out): the first and last ones, and
+    those on either side of the slices' border."""
+    batch, c, w = 65535, 257, 257
+    if torch.cuda.mem_get_info()[0] < 24 << 30:
+        pytest.skip("needs 17 GB of free memory")
+    x = torch.empty(batch, c * w, dtype=torch.float16, device="cuda")
+    x[:] = ((torch.arange(c * w, device="cuda") * 7919) % 10007 - 5000).half()
+    x[:, 0] = (torch.arange(batch, device="cuda") % 2048).half()  # images differ
+    y = torch.full_like(x, float("nan"))
+    torch.cuda.synchronize()
+    ops.pool(ops.POOL_MAX, x.data_ptr(), y.data_ptr(), c, 1, w, 3, 1, 1, batch)
+    torch.cuda.synchronize()
+    edge = (((1 << 24) - 1) // c)  # images a launch holds
+    for i in (0, 1, edge - 1, edge, edge + 1, batch - 1):
+        p = torch.nn.functional.pad(x[i].view(c, w).float(), (1, 1), value=float("-inf"))
+        ref = torch.maximum(torch.maximum(p[:, :-2], p[:, 1:-1]), p[:, 2:])
+        assert torch.equal(y[i].view(c, w).float(), ref), f"image {i}"
+    assert not torch.isnan(y[:, ::1001]).any()
 
 
 @pytest.mark.parametrize("cin,cout,h,w,res,off", [
