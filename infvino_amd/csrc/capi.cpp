@@ -84,6 +84,13 @@ ivh::ConvSpec conv_spec(const ivh_conv_desc * d, bool gemv)
   return s;
 }
 
+// A 1x1 conv of one-pixel planes is an FC: [batch][cin] rows, packed and run as ivh_gemv_f16 does
+// whichever entry point it is given to.
+bool one_pixel(const ivh_conv_desc * d)
+{
+  return d && d->h == 1 && d->w == 1 && d->k == 1 && d->pad == 0 && d->groups == 1 && !d->channels_last;
+}
+
 ivh::View tensor_view(const void * ptr, int C, int H, int W, bool nhwc)
 {
   ivh::View v;
@@ -109,7 +116,8 @@ void check_batch(int batch)
 void run_conv(const ivh_conv_desc * d, bool gemv, bool dw_only, const void * x, const void * packed, const void * res,
               void * y, int batch, void * stream)
 {
-  const ivh::ConvSpec s = conv_spec(d, gemv);
+  const bool rows = gemv || one_pixel(d);
+  const ivh::ConvSpec s = conv_spec(d, rows);
   const ivh::ConvPacking pk = ivh::conv_packing(s);
   if (dw_only && pk.family != ivh::kFamDw) throw std::invalid_argument("not a depthwise conv (groups == cin == cout, k 3/5)");
   if (gemv && (s.H != 1 || s.W != 1 || s.K != 1 || s.G != 1 || s.P != 0)) throw std::invalid_argument("gemv descriptor");
@@ -124,7 +132,7 @@ void run_conv(const ivh_conv_desc * d, bool gemv, bool dw_only, const void * x, 
   p.x = tensor_view(x, s.Cin, s.H, s.W, s.x_nhwc);
   p.y = tensor_view(y, s.Cout, p.Ho, p.Wo, s.x_nhwc);
   if (res) p.r = tensor_view(res, s.Cout, p.Ho, p.Wo, s.x_nhwc);
-  if (gemv) {  // [batch][n] rows: one pixel per image, presented channels-last
+  if (rows) {  // [batch][n] rows: one pixel per image, presented channels-last
     for (ivh::View * v : {&p.x, &p.y, &p.r}) {
       if (!v->ptr) continue;
       const int C = v == &p.x ? s.Cin : s.Cout;
@@ -409,7 +417,7 @@ int ivh_conv_packed_bytes(const ivh_conv_desc * d, size_t * bytes)
 {
   return guard([&] {
     if (!bytes) throw std::invalid_argument("null bytes");
-    *bytes = ivh::conv_packing(conv_spec(d, d && d->h == 1 && d->w == 1 && d->k == 1)).bytes;
+    *bytes = ivh::conv_packing(conv_spec(d, one_pixel(d))).bytes;
   });
 }
 
@@ -417,7 +425,7 @@ int ivh_pack_conv_weights(const ivh_conv_desc * d, const uint16_t * w_host, cons
                           void * packed_dev)
 {
   return guard([&] {
-    const ivh::ConvSpec s = conv_spec(d, d && d->h == 1 && d->w == 1 && d->k == 1);
+    const ivh::ConvSpec s = conv_spec(d, one_pixel(d));
     if (!w_host || !packed_dev) throw std::invalid_argument("null operand");
     if (s.has_bias && !bias_host) throw std::invalid_argument("has_bias set but bias is null");
     const ivh::ConvPacking pk = ivh::conv_packing(s);

@@ -122,6 +122,31 @@ def test_abi_gemv(n_in, n_out, act):
         assert _ok(y[b], ref, f"gemv {n_in}->{n_out} image {b}")
 
 
+@pytest.mark.parametrize("n_in,n_out,res,pad", [(64, 10, False, 0), (576, 1000, True, 0), (100, 37, True, 0),
+                                                (16, 24, False, 1)])
+def test_abi_conv2d_one_pixel_planes(n_in, n_out, res, pad):
+    """ivh_conv2d_f16 on planes of one pixel (a squeeze-and-excite layer's 1x1 conv) reads the
+    packing that the descriptor got."""
+    B = 5
+    rng = np.random.default_rng(n_in)
+    d = ops.conv_desc(n_in, n_out, 1, 1, 1, 1, pad, act=ops.ACT_HSIGMOID, channels_last=False)
+    ho, wo = ops.conv_out_dims(d)
+    no = n_out * ho * wo
+    x = O.f2h(rng.random(B * n_in).astype(np.float32))
+    wt = O.f2h((rng.standard_normal(n_out * n_in) * np.sqrt(2.0 / n_in)).astype(np.float32))
+    bias = O.f2h((rng.standard_normal(n_out) * 0.01).astype(np.float32))
+    r = O.f2h(rng.random(B * no).astype(np.float32)) if res else None
+    packed = _pack(d, wt, bias)
+    xd, yd, rd = _dev(x), _dev(np.full(B * no + 8, NAN16, np.uint16)), _dev(r) if res else None
+    ops.conv2d(d, xd.data_ptr(), packed.data_ptr(), rd.data_ptr() if res else None, yd.data_ptr(), B)
+    y = _host(yd)
+    assert np.all(y[B * no:] == NAN16)
+    for b in range(B):
+        ref = O.conv2d(x[b * n_in:(b + 1) * n_in], wt, bias, None if r is None else r[b * no:(b + 1) * no], n_in, 1, 1,
+                       n_out, 1, 1, pad, 1, ho, wo, ops.ACT_HSIGMOID, O.F32, 1 if pad == 0 else 0)
+        assert _ok(y[b * no:(b + 1) * no], ref, f"one pixel {n_in}->{n_out} image {b}")
+
+
 def test_abi_eltwise():
     B, n = 2, 4000
     rng = np.random.default_rng(7)
