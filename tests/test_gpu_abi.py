@@ -319,7 +319,9 @@ def test_abi_pointwise_planes(cin, cout, h, w, res, off):
     (8, 12, 6, 6, 5, 1, 3, False),        # four taps a chunk
     (128, 192, 40, 40, 3, 1, 1, True),    # 64 x 32 tiles, eight waves
     (64, 64, 40, 40, 3, 1, 8, True),      # 64 x 64 tiles, pixels of two images in a tile
-    (60, 130, 39, 39, 1, 1, 3, False),    # the same with a half-empty last channel tile, Cin % 8
+    (124, 130, 39, 39, 1, 1, 3, False),   # the same with a nearly empty last channel tile, Cin % 8
+    (60, 130, 39, 39, 1, 1, 3, False),    # two chunks of channels: the implicit GEMM
+    (256, 192, 25, 25, 1, 1, 3, True),    # 32 x 32 tiles, two chunks a wave, a partial last pixel tile
     (256, 64, 3, 3, 1, 2, 5, False),      # stride 2 pointwise
 ])
 def test_abi_small_grid_conv(cin, cout, h, w, k, s, B, res):
@@ -407,7 +409,8 @@ def test_abi_softmax_rows(axis):
 @pytest.mark.parametrize("cin,cout,h,w,k,s,B,res", [
     (256, 128, 40, 40, 1, 1, 8, True),    # K halves of four steps, 128-channel tiles, residual
     (72, 200, 29, 31, 3, 2, 40, False),   # an odd step count over the halves, partial tiles both ways
-    (64, 64, 80, 80, 3, 2, 8, False),     # 64-channel tiles
+    (64, 64, 80, 80, 3, 2, 11, False),    # 64-channel tiles, K halves with taps
+    (64, 64, 80, 80, 3, 2, 8, False),     # ... and a batch that the small-grid kernel takes
     (264, 40, 33, 35, 1, 1, 20, True),    # the same, 9 steps, 40 of 64 channels
     (40, 256, 53, 53, 1, 1, 7, False),    # whole K: two steps, the second ragged
     (32, 136, 61, 59, 3, 2, 40, True),    # whole K with taps, a second channel tile of 8

@@ -524,6 +524,23 @@ def test_tile_configs(tmp_path, cin, cout, hw, k, batch, want):
     _check_f32(path, batch, lo=-1.0, ref_mode=False, flags=ia.IVH_FLAG_NO_PIPE)
 
 
+@pytest.mark.parametrize("cin,cout,hw,k,s,batch,splits", [
+    (512, 100, 20, 1, 1, 21, 4),   # K step 64, 100 of 128 channels
+    (500, 100, 20, 1, 1, 24, 4),   # Cin % 8
+    (256, 100, 20, 3, 2, 90, 6),   # taps
+])
+def test_split_k_over_work_groups(tmp_path, cin, cout, hw, k, s, batch, splits):
+    """Channels-last convs whose K range is split over work-groups (fp32 partials in memory and a
+    fixed-order reduce): mid-size grids whose channel counts the DMA-fed build does not take."""
+    path, _ = pw.single_conv(str(tmp_path), cin, cout, hw, hw, k=k, s=s, act=pw.ACT_SILU, pre_relu=True, post_relu=True)
+    tag = _conv_tags(path, batch)[0].split()
+    assert tag[0] == "conv_igemm_sk" and f"ksplit={splits}" in tag, tag
+    got = _check_f32(path, batch, lo=-1.0, ref_mode=False)
+    _, _, nosplit = _run(path, batch, lo=-1.0, flags=ia.IVH_FLAG_NO_SPLITK)
+    mean_rel, max_rel, _, _ = O.rel_errors(O.h2f(got[0]), O.h2f(nosplit[0]))
+    assert mean_rel < 1e-3 and max_rel < 5e-3
+
+
 @pytest.mark.parametrize("cin,cout,hw,k,s,batch", [
     (256, 256, 20, 3, 1, 1),   # batch 1: 8 output tiles, 72 K tiles -> split-K
     (128, 51, 40, 3, 1, 1),
@@ -532,7 +549,7 @@ def test_tile_configs(tmp_path, cin, cout, hw, k, batch, want):
     (128, 256, 40, 3, 2, 3),
 ])
 def test_split_k(tmp_path, cin, cout, hw, k, s, batch):
-    """Small-M / long-K convs take the split-K path (partials + fixed-order reduce)."""
+    """Small-M / long-K convs split K over the waves of a work-group (the small-grid kernel)."""
     path, _ = pw.single_conv(str(tmp_path), cin, cout, hw, hw, k=k, s=s, act=pw.ACT_SILU, pre_relu=True)
     assert _conv_kernel(path, batch) == "conv_igemm_sk"
     assert _conv_kernel(path, batch, ia.IVH_FLAG_NO_SPLITK) != "conv_igemm_sk"
@@ -914,9 +931,10 @@ def _upcat_plan(d, ca, cb, cout, H, W, reuse_a):
 ])
 def test_upsample_concat_fused(tmp_path, ca, cb, cout, H, W, batch, reuse_a, fused):
     """The 1x1 conv reads the upsampled channels from the resize's input: same bits as the
-    materialised concat (the same implicit GEMM, the same values in the same LDS rows)."""
+    materialised concat (on the small-grid kernel where the output is an internal tensor, on the
+    implicit GEMM where it is the graph's, in planes)."""
     path = _upcat_plan(tmp_path, ca, cb, cout, H, W, reuse_a)
-    fl = ia.IVH_FLAG_NO_PW  # both runs on the implicit GEMM, which the fused conv always uses
+    fl = ia.IVH_FLAG_NO_PW  # both runs on the implicit GEMM's family, which the fused conv always uses
     tags = _conv_tags(path, batch, fl)
     assert sum("upsample-concat" in t for t in tags) == (1 if fused else 0), tags
     assert ("resize_nn" in _kernels(path, batch, fl)) == (not fused)
@@ -925,6 +943,31 @@ def test_upsample_concat_fused(tmp_path, ca, cb, cout, H, W, batch, reuse_a, fus
     _, _, ref = _run(path, batch, lo=-1.0, flags=fl | ia.IVH_FLAG_NO_FUSE_UPSAMPLE)
     assert np.array_equal(got[0], ref[0])
     _check_f32(path, batch, lo=-1.0, ref_mode=False, flags=fl)
+
+
+@pytest.mark.parametrize("ca,cb,cout,H,W,batch,want", [
+    (128, 64, 64, 40, 40, 4, "dma"),             # 192 -> 64 at 80x80: whole K, 64-channel tiles
+    (128, 64, 64, 40, 40, 12, "dma"),
+    (256, 128, 128, 20, 20, 8, "dma k-halves"),  # 384 -> 128 at 40x40: K halves, 128-channel tiles
+    (256, 128, 128, 20, 20, 40, "dma"),
+    (192, 64, 72, 13, 11, 30, "dma k-halves"),   # odd maps, 72 of 128 channels
+    (256, 128, 128, 20, 20, 64, ""),             # more tiles than the DMA-fed build takes: conv_igemm_kernel
+])
+def test_upsample_concat_large(tmp_path, ca, cb, cout, H, W, batch, want):
+    """The upsample-concat input of the DMA-fed implicit GEMM and of the plain one: same bits as the
+    materialised concat, and the first and last image against the oracle."""
+    path = _upcat_plan(tmp_path, ca, cb, cout, H, W, True)  # the conv's output is an internal tensor
+    fl = ia.IVH_FLAG_NO_PW
+    tag = next(t.split() for t in _conv_tags(path, batch, fl) if "upsample-concat" in t)
+    assert tag[0] == "conv_igemm" and all((f in tag) == (f in want.split()) for f in ("dma", "k-halves")), tag
+    p, x, got = _run(path, batch, lo=-1.0, flags=fl)
+    _, _, ref = _run(path, batch, lo=-1.0, flags=fl | ia.IVH_FLAG_NO_FUSE_UPSAMPLE)
+    assert np.array_equal(got[0], ref[0])
+    n = p.numel(p.input_name)
+    want = O.run_plan(p, np.concatenate([x[:n], x[-n:]]), 2)[0].reshape(2, -1)
+    for i, j in ((0, 0), (batch - 1, 1)):
+        mean_rel, max_rel, _, _ = O.rel_errors(O.h2f(got[0].reshape(batch, -1)[i]), O.h2f(want[j]))
+        assert mean_rel < F32_MEAN and max_rel < F32_MAX, (i, mean_rel, max_rel)
 
 
 def _head_plan(d, cin, H, W, widths=(51, 64, 64)):

@@ -201,6 +201,34 @@ def test_launch_tags(tmp_path, shape, head, detail, flags):
     assert tag.startswith(head) and detail in tag.split(), tag
 
 
+@pytest.mark.parametrize("cin,cout,h,w,k,s,batch,want", [
+    # the small-grid kernel: pixels x channels of a tile, waves
+    (256, 256, 20, 20, 3, 1, 1, "bm=32 bn=32 waves=8"), (128, 100, 13, 11, 3, 2, 2, "bm=32 bn=32 waves=8"),
+    (100, 200, 15, 15, 3, 2, 7, "bm=32 bn=32 waves=8 cin-ragged"), (40, 33, 7, 9, 1, 1, 1, "bm=32 bn=32 waves=4"),
+    (8, 12, 6, 6, 5, 1, 3, "bm=32 bn=32 waves=4"), (256, 192, 25, 25, 1, 1, 3, "bm=32 bn=32 waves=4"),
+    (128, 192, 40, 40, 3, 1, 1, "bm=64 bn=32 waves=8"), (124, 130, 39, 39, 1, 1, 3, "bm=64 bn=64 waves=4 cin-ragged"),
+    (64, 64, 80, 80, 3, 2, 8, "bm=64 bn=64 waves=4"),
+    # the DMA-fed implicit GEMM, whole K and in halves, and the streaming 1x1 kernel
+    (256, 128, 40, 40, 1, 1, 8, "bn=128 dma k-halves"), (72, 200, 29, 31, 3, 2, 40, "bn=128 dma k-halves"),
+    (64, 64, 80, 80, 3, 2, 11, "bn=64 dma k-halves"), (264, 40, 33, 35, 1, 1, 20, "bn=64 dma k-halves"),
+    (40, 256, 53, 53, 1, 1, 7, "bn=128 dma"), (32, 136, 61, 59, 3, 2, 40, "bn=128 dma"),
+    (192, 128, 64, 64, 1, 1, 16, "streamed"), (136, 72, 81, 83, 1, 1, 11, "streamed"),
+    (384, 104, 90, 91, 1, 1, 13, "streamed"),
+    # the implicit GEMM itself, whole and with partial sums in memory
+    (60, 130, 39, 39, 1, 1, 3, "bn=128 ksplit=1 cin-ragged"), (512, 100, 20, 20, 1, 1, 21, "bn=128 ksplit=4"),
+])
+def test_implicit_gemm_routes(tmp_path, cin, cout, h, w, k, s, batch, want):
+    """Which of the implicit-GEMM kernels, and which build of it, runs the shapes of the GPU tests."""
+    path, _ = pw.single_conv(str(tmp_path), cin, cout, h, w, k=k, s=s, act=pw.ACT_SILU, pre_relu=True, post_relu=True)
+    m = ia.PlanModel(path, 0, batch, DRY)
+    m.run(batch)
+    tag = next(m.nodeTag(i) for i in range(m.nodeCount()) if m.nodeInfo(i)["op"].startswith("conv")).split()
+    m.close()
+    assert set(want.split()) <= set(tag), tag
+    for f in ("dma", "k-halves", "streamed", "cin-ragged"):
+        assert (f in tag) == (f in want.split()), tag
+
+
 def test_depthwise_tile_for_every_channel_count(tmp_path):
     """The depthwise planner finds a tile within the kernel's limits (256 lanes, 4096 LDS pieces,
     1024 weight pieces) for every channel count, those whose groups of 8 have no divisor that
