@@ -739,7 +739,9 @@ __global__ void __launch_bounds__(256) dw_strip_kernel(const ConvParams p, FastD
 // Any-layout depthwise: one lane = one output pixel of one channel plane, grid (pixel
 // blocks, channel, image) so that the channel's weights are wave-uniform (scalar loads) and,
 // on NCHW tensors, neighbouring lanes read neighbouring pixels.  Same tap order and roundings
-// as the channels-last kernels: act(sum + b), one fp16 rounding, then the residual.
+// as the channels-last kernels: act(sum + b), one fp16 rounding, then the residual.  FAST: their
+// activation formulas too, for convs that take those kernels at other batch sizes.
+template <bool FAST>
 __global__ void __launch_bounds__(256) dw_generic_kernel(const ConvParams p, FastDiv d_wo)
 {
   const int HWo = p.Ho * p.Wo;
@@ -758,7 +760,23 @@ __global__ void __launch_bounds__(256) dw_generic_kernel(const ConvParams p, Fas
       acc += vld(p.x, b, c, (long)iy * p.W + ix) * W[(ky * p.K + kx) * p.Cin + c];
     }
   }
-  float v = (float)(_Float16)act_f(acc + (p.bias ? p.bias[c] : 0.0f), p.act);
+  acc += p.bias ? p.bias[c] : 0.0f;
+  _Float16 h;
+  if (FAST) {
+    float v;
+    switch (p.act) {
+    case kActSiLU: v = act_fast<kActSiLU>(acc); break;
+    case kActReLU: v = act_fast<kActReLU>(acc); break;
+    case kActHSwish: v = act_fast<kActHSwish>(acc); break;
+    case kActHSigmoid: v = act_fast<kActHSigmoid>(acc); break;
+    case kActSigmoid: v = act_fast<kActSigmoid>(acc); break;
+    default: v = acc; break;
+    }
+    h = round_f16(v);
+  } else {
+    h = (_Float16)act_f(acc, p.act);
+  }
+  float v = (float)h;
   if (p.r.ptr) v += vld(p.r, b, c, hw);
   vst(p.y, b, c, hw, v);
 }
@@ -1055,7 +1073,9 @@ void launch_dwconv(const ConvParams & p, hipStream_t s)
       else hipLaunchKernelGGL((dw_nchw_kernel<5, 2, PX>), g, dim3(256), 0, s, p, f, fp);
     } else {
       const dim3 grid(nblk((long)p.Ho * p.Wo, 256), (unsigned)p.Cin, (unsigned)p.batch);
-      hipLaunchKernelGGL(dw_generic_kernel, grid, dim3(256), 0, s, p, fastdiv_make((unsigned)p.Wo));
+      const FastDiv f = fastdiv_make((unsigned)p.Wo);
+      if (dwconv_vectorizable(p)) hipLaunchKernelGGL(dw_generic_kernel<true>, grid, dim3(256), 0, s, p, f);
+      else hipLaunchKernelGGL(dw_generic_kernel<false>, grid, dim3(256), 0, s, p, f);
     }
     return;
   }

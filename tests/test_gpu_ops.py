@@ -659,12 +659,11 @@ def test_depthwise_kernel_check_shapes(tmp_path, c, h, w, k, s, p, act):
 @pytest.mark.parametrize("c,hw,k,s,batches", [
     (16, 112, 3, 2, (1, 6)), (64, 80, 3, 1, (1, 3)), (240, 14, 5, 1, (1, 9)), (576, 7, 5, 1, (1, 5)),
     (88, 28, 3, 1, (2, 4)), (120, 33, 5, 2, (1, 3)), (8, 61, 5, 1, (1, 2)), (40, 45, 3, 2, (3, 1)),
-    (96, 56, 5, 2, (48, 1))])  # batch 48: the 5x5 stride-2 strip kernel; batch 1: tiled
+    (96, 56, 5, 2, (48, 1))])
 def test_depthwise_tiles(tmp_path, c, hw, k, s, batches):
-    """Channels-last depthwise over tile grids with ragged right and bottom edges, several
-    channel tiles and sizes whose tile choice (or kernel) changes with the batch: every batch
-    size agrees with the oracle, and image 0 is bit-identical across batch sizes (the
-    per-pixel sum order does not depend on the tile or kernel)."""
+    """Depthwise from an internal channels-last tensor into the graph's planar output (the any-layout
+    kernel): every batch size agrees with the oracle, and image 0 is bit-identical across batch
+    sizes.  test_depthwise_channels_last_batches has the tiled and strip kernels."""
     path, _ = pw.single_conv(str(tmp_path), c, c, hw, hw, k=k, s=s, groups=c, act=pw.ACT_HSWISH, pre_relu=True)
     outs = []
     for b in batches:
@@ -673,6 +672,38 @@ def test_depthwise_tiles(tmp_path, c, hw, k, s, batches):
     n0 = outs[0].size // batches[0]
     for o, b in zip(outs[1:], batches[1:]):
         assert np.array_equal(o[:n0], outs[0][:n0])
+
+
+@pytest.mark.parametrize("c,hw,k,s,act,batches,kernels", [
+    (16, 112, 3, 2, 3, (1, 6), ("tile", "tile")), (64, 80, 3, 1, 1, (1, 3), ("tile", "tile")),
+    (240, 14, 5, 1, 3, (1, 9), ("tile", "tile")), (96, 56, 5, 2, 3, (48, 1), ("strip", "tile")),
+    (70, 56, 5, 2, 1, (60, 1), ("strip", "tile")),                    # a partial last channel group
+    (147, 40, 3, 1, 5, (1, 8), ("tile", "tile")), (41, 28, 5, 1, 4, (1, 40), ("tile", "tile")),
+    (33, 20, 3, 1, 1, (1, 8, 64), ("tile", "generic", "tile")),       # ... and little work: the any-layout kernel
+    (15, 28, 5, 2, 3, (1, 30, 600), ("tile", "generic", "tile")), (7, 7, 3, 1, 4, (1, 64), ("tile", "generic")),
+])
+def test_depthwise_channels_last_batches(tmp_path, c, hw, k, s, act, batches, kernels):
+    """Channels-last depthwise convs inside a plan on the tiled, strip and any-layout kernels: each
+    batch size against the oracle (first and last image), and image 0 bit-identical across batch
+    sizes (one sum order, one activation formula and one rounding in all three)."""
+    path, _ = pw.single_conv(str(tmp_path), c, c, hw, hw, k=k, s=s, groups=c, act=act, pre_relu=True, post_relu=True)
+    plan, first = O.Plan.load(path), None
+    n = plan.numel(plan.input_name)
+    x = O.f2h((np.random.default_rng(c).random(n * max(batches), dtype=np.float32) * 2 - 1))
+    for b, want in zip(batches, kernels):
+        m = ia.PlanModel(path, 0, b)
+        m.setInput(x[:n * b], b)
+        m.run(b)
+        tag = next(m.nodeTag(i) for i in range(m.nodeCount()) if m.nodeInfo(i)["kernel"] == "dwconv")
+        assert tag.split()[1] == want, tag
+        got = m.readOutput(0, b).reshape(b, -1)
+        m.close()
+        ref = O.run_plan(plan, np.concatenate([x[:n], x[(b - 1) * n:b * n]]), 2)[0].reshape(2, -1)
+        for i, j in ((0, 0), (b - 1, 1)):
+            mean_rel, max_rel, _, _ = O.rel_errors(O.h2f(got[i]), O.h2f(ref[j]))
+            assert mean_rel < F32_MEAN and max_rel < F32_MAX, (b, i, mean_rel, max_rel)
+        first = got[0] if first is None else first
+        assert np.array_equal(got[0], first), f"batch {b}: {(got[0] != first).sum()} values"
 
 
 def _small_plan(d, build):
