@@ -1,10 +1,10 @@
 // The implicit GEMM of conv_mfma.hip fed through LDS by DMA, gfx950 fp16 MFMA: the channels-last
 // 1x1 and strided convs whose grids fill the chip.
 //
-// Same tiles (128 pixels x 64 or 128 channels, 4 waves), operands and K order as
-// conv_igemm_kernel, and the same results.  That kernel carries both operands through
-// registers into LDS: as many LDS writes as reads, 16 to 32 registers a step.  Here buffer
-// loads with the LDS flag copy a step of 32 channels (128 rows of 64 bytes per operand,
+// Same tiles (128 pixels x 64 or 128 channels, 4 waves), operands, K order and rounding as
+// conv_igemm_kernel, and so the same results with the whole K range (KG = 1).  That kernel
+// carries both operands through registers into LDS: as many LDS writes as reads, 16 to 32
+// registers a step.  Here buffer loads with the LDS flag copy a step of 32 channels (128 rows of 64 bytes per operand,
 // swizzled as in conv_small.hip) into one of three stages, two steps ahead; a wave waits for
 // its own copies of the step (a compile-time vmcnt count), one barrier publishes every wave's
 // and retires the stage the next copies overwrite; the fragments are read before the next
@@ -16,9 +16,9 @@
 // the same), so with at most one work-group per CU eight waves halve the K range between
 // two groups with stages of their own (KG = 2) and add their sums through LDS at the end.
 // Measured on MI355X as single calls, against conv_igemm_kernel: 128->256 3x3 stride 2 at 40x40,
-// batch 8 / 16 / 64 (KG 2, 2, 1): 20.6 -> 14.1, 21.2 -> 15.7, 30.5 -> 29.8 us; 64->64 at 80x80
-// stride 2, batch 8 (KG 2): 11.5 -> 7.5 us; 512->256 1x1 at 20x20, batch 8 / 64 (KG 2, 1):
-// 12.9 -> 9.1, 18.3 -> 17.5 us; 384->128 1x1 at 40x40, batch 32 (KG 1): 18.7 -> 16.4 us.
+// batch 16 / 64 (KG 2, 1): 21.2 -> 15.7, 30.5 -> 29.8 us; 64->64 at 80x80 stride 2, batch 11
+// (KG 2): 11.6 -> 7.9 us; 512->256 1x1 at 20x20, batch 64 (KG 1): 18.3 -> 17.5 us; 384->128 1x1 at
+// 40x40, batch 32 (KG 1): 18.7 -> 16.4 us.
 #include "conv_common.hpp"
 #include "kernels.hpp"
 

@@ -1,6 +1,6 @@
 // Implicit-GEMM convolution for grids that cannot fill the chip (one image or a few, deep
 // maps, the classifier's GEMV) on gfx950 fp16 MFMA: the K range is split over the waves of a
-// work-group and no operand passes through LDS.
+// work-group, and no barrier stands in the K loop.
 //
 // Same math and operands as conv_igemm_kernel (conv_mfma.hip): M = output pixels of all
 // images, N = output channels, K = (ky, kx, ci) in 8-channel pieces, weights in the
@@ -331,9 +331,11 @@ bool small_views_ok(const ConvParams & p)
 //   384->128 1x1 at 40x40, batch 1 / 2 / 4 / 8: 4.9 vs 11.7, 5.5 vs 11.8, 7.5 vs 11.9, 13.2
 //     (400) vs 13.5 us
 //   64->64 1x1 at 80x80, batch 1 / 2: 5.1 vs 5.9, 6.1 (config 3, two chunks) vs 5.6 us
-// Config 0 gives eight waves a K range of at least two chunks each.  Config 3 amortises its
-// longer tile over at least four chunks per wave pair (K >= 256 for 1x1, any 3x3 that gets
-// here is longer).
+// Config 0 gives eight waves a K range of at least two chunks each.  Config 3 gives its four
+// waves at least one each (K > 96 in 1x1 convs; any 3x3 that gets here is longer).  1x1 at that
+// end, against the DMA-fed implicit GEMM: 104->128 at 40x40, batch 4: 6.0 vs 7.8 us, 192->256 at
+// 40x40, batch 2: 6.5 vs 8.2; with 33 to 64 outputs that build's smaller tile is the faster one
+// (128->64 at 40x40, batch 8: 5.9 vs 5.3 us, 320->64: 7.0 vs 5.8), which the rule does not use.
 int small_plan(const ConvParams & p)
 {
   if (!small_views_ok(p)) return 0;

@@ -1,7 +1,7 @@
 // 1x1 stride-1 convs with 64 < Cout <= 128 and 128 < Cin <= 384 on large channels-last maps,
 // gfx950 fp16 MFMA: weights in registers, pixels streamed through LDS by DMA, persistent.
 //
-// Same operands, K order and results as conv_igemm_kernel.  Bound: HBM.  As 128 x 128 tiles such a
+// Same operands, K order, rounding and results as conv_igemm_kernel.  Bound: HBM.  As 128 x 128 tiles such a
 // layer is one round of work-groups that all load, then compute, then store (800 tiles of
 // 40x40 maps at batch 64), so the memory idles between the phases and each tile fetches the
 // weights again.  Here two work-groups of four waves per CU walk contiguous shares of the

@@ -1861,8 +1861,8 @@ __global__ void __launch_bounds__(256) softmax_pieces_kernel(const SmallParams q
   for (int i = 0; i < NP; ++i)
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      ex[i][e] = __expf((float)v[i][e] - m);  // the filler past the row's end adds exp(-inf) = 0
-      s += (sub + L * i) * 8 + e < n ? ex[i][e] : 0.0f;
+      ex[i][e] = __expf((float)v[i][e] - m);
+      s += (sub + L * i) * 8 + e < n ? ex[i][e] : 0.0f;  // the filler past the row's end left out
     }
 #pragma unroll
   for (int off = L / 2; off > 0; off >>= 1) s += __shfl_xor(s, off);
