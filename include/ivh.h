@@ -127,6 +127,10 @@ int ivh_set_input_f32(ivh_model * m, const float * host, int batch);
 int ivh_set_input_f32_noalloc(ivh_model * m, const float * host, int batch);
 int ivh_run(ivh_model * m, int batch);
 int ivh_sync(ivh_model * m);
+/* output i as fp16, or converted exactly to f32; both wait for the model's runs.  Large fp16 reads
+   into pageable memory (2 MB and more) and f32 reads pass through pinned host memory that the
+   model keeps (as much as its largest read, at most 16 MB), and reads of 8 MB and more are copied
+   out by up to eight host threads that end with the call. */
 int ivh_read_output_f16(ivh_model * m, int i, uint16_t * host, int batch);
 int ivh_read_output_f32(ivh_model * m, int i, float * host, int batch);
 /* any declared tensor, as NCHW fp16; returns IVH_ERR_INVALID for an unknown name */
