@@ -2777,15 +2777,16 @@ bool Model::ringRead(char * dst, size_t bytes, const std::function<void(char *, 
   return true;
 }
 
-// pinned (or device-visible) host memory, which the copy engine reaches without a detour
-static bool pinned_host(const void * p)
+// Memory that the runtime knows: pinned host memory, which the copy engine reaches without a
+// detour, and managed or device memory, which its copy takes and a host copy may not.
+static bool known_memory(const void * p)
 {
   hipPointerAttribute_t a{};
   if (hipPointerGetAttributes(&a, p) != hipSuccess) {
-    (void)hipGetLastError();  // memory the runtime does not know
+    (void)hipGetLastError();
     return false;
   }
-  return a.type == hipMemoryTypeHost || a.type == hipMemoryTypeManaged;
+  return a.type != hipMemoryTypeUnregistered;
 }
 
 void Model::readOutputF16(int i, uint16_t * host, int batch)
@@ -2801,7 +2802,7 @@ void Model::readOutputF16(int i, uint16_t * host, int batch)
   // MB).  Pinned destinations take the runtime's one copy: 75 against 130 us for 3.8 MB, 1.06
   // against 1.43 ms for 60 MB.
   const size_t bytes = (size_t)t.numel * 2 * batch;
-  if ((batch == 1 || v.img == t.numel) && bytes >= ((size_t)2 << 20) && !dry_ && !pinned_host(host)) {
+  if ((batch == 1 || v.img == t.numel) && bytes >= ((size_t)2 << 20) && !dry_ && !known_memory(host)) {
     const char * src = reinterpret_cast<const char *>(v.ptr);
     auto fill = [&](char * pin, size_t off, size_t len) {
       launch_copy_out(src + off, pin, (long)len, stream_);

@@ -516,7 +516,8 @@ def test_abi_stem_planes(cin, cout, h, w, B, act):
 
 def test_readback_into_pinned_memory(tmp_path):
     """A pinned destination: the same values, and, as one copy without the ring's detour, no
-    slower than the same read into pageable memory."""
+    slower than the same read into pageable memory.  A device destination is the runtime's
+    business too: written or refused, never touched by the host."""
     hw, batch = 1024, 8
     n = hw * hw
     path = tmp_path / "io.plan"
@@ -535,6 +536,10 @@ def test_readback_into_pinned_memory(tmp_path):
             best = min(best, time.perf_counter() - t0)
         assert np.array_equal(buf.numpy().view(np.uint16), x)
         took.append(best)
+    dev = torch.zeros(n * batch, dtype=torch.int16, device="cuda")
+    torch.cuda.synchronize()
+    if ia.lib().ivh_read_output_f16(m._h, 0, dev.data_ptr(), batch) == 0:  # the runtime's copy takes it
+        assert np.array_equal(dev.cpu().numpy().view(np.uint16), x)
     print(f"16 MB: pinned {took[0] * 1e6:.0f} us, pageable {took[1] * 1e6:.0f} us")
     m.close()
     assert took[0] < took[1]
