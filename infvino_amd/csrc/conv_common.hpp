@@ -162,7 +162,8 @@ __device__ __forceinline__ void load_bias(const ConvParams & p, int n0, float (&
 
 // Epilogue phase 1: bias + activation (compile-time code) in fp32, one rounding to fp16,
 // tile into LDS as [pixel][channel] (NHWC output) or [channel][pixel] (NCHW output).
-template <int ACT, int MB, int WGM, int WGN, int TM, int TN>
+// ROUND: with round_f16, as the kernels that share this one's sums.
+template <bool ROUND, int ACT, int MB, int WGM, int WGN, int TM, int TN>
 __device__ __forceinline__ void stage_tile(typename Mf<MB>::acc_t (&acc)[TN][TM], const float (&bv)[TN][Mf<MB>::NV],
                                            _Float16 * lds, bool nhwc)
 {
@@ -182,7 +183,10 @@ __device__ __forceinline__ void stage_tile(typename Mf<MB>::acc_t (&acc)[TN][TM]
         const int cl = wn * TN * MB + tn * MB + F::row(lane, v4);
         h4 hv;
 #pragma unroll
-        for (int k = 0; k < 4; ++k) hv[k] = round_f16(act_fast<ACT>(acc[tn][tm][v4 + k] + bv[tn][v4 + k]));
+        for (int k = 0; k < 4; ++k) {
+          const float v = act_fast<ACT>(acc[tn][tm][v4 + k] + bv[tn][v4 + k]);
+          hv[k] = ROUND ? round_f16(v) : (_Float16)v;
+        }
         if (nhwc) {
           *reinterpret_cast<h4 *>(lds + pl * (BN + 8) + cl) = hv;
         } else {
@@ -201,7 +205,7 @@ __device__ __forceinline__ void stage_tile(typename Mf<MB>::acc_t (&acc)[TN][TM]
 // With p.ksplit > 1 the fp32 partials go to the workspace [kz][co][pixel] instead.
 // tile_epilogue_bv takes the bias values already loaded (load_bias), for kernels whose
 // loads of the next tile are in flight during the epilogue.
-template <int MB, int WGM, int WGN, int TM, int TN, class PixFn>
+template <bool ROUND, int MB, int WGM, int WGN, int TM, int TN, class PixFn>
 __device__ __forceinline__ void tile_epilogue_bv(typename Mf<MB>::acc_t (&acc)[TN][TM],
                                                  const float (&bv)[TN][Mf<MB>::NV], const ConvParams & p,
                                                  _Float16 * lds, int n0, int kz, PixFn pix)
@@ -235,12 +239,12 @@ __device__ __forceinline__ void tile_epilogue_bv(typename Mf<MB>::acc_t (&acc)[T
 
   const bool nhwc = p.y.layout == kNHWC;
   switch (p.act) {
-  case kActSiLU: stage_tile<kActSiLU, MB, WGM, WGN, TM, TN>(acc, bv, lds, nhwc); break;
-  case kActReLU: stage_tile<kActReLU, MB, WGM, WGN, TM, TN>(acc, bv, lds, nhwc); break;
-  case kActHSwish: stage_tile<kActHSwish, MB, WGM, WGN, TM, TN>(acc, bv, lds, nhwc); break;
-  case kActHSigmoid: stage_tile<kActHSigmoid, MB, WGM, WGN, TM, TN>(acc, bv, lds, nhwc); break;
-  case kActSigmoid: stage_tile<kActSigmoid, MB, WGM, WGN, TM, TN>(acc, bv, lds, nhwc); break;
-  default: stage_tile<kActNone, MB, WGM, WGN, TM, TN>(acc, bv, lds, nhwc); break;
+  case kActSiLU: stage_tile<ROUND, kActSiLU, MB, WGM, WGN, TM, TN>(acc, bv, lds, nhwc); break;
+  case kActReLU: stage_tile<ROUND, kActReLU, MB, WGM, WGN, TM, TN>(acc, bv, lds, nhwc); break;
+  case kActHSwish: stage_tile<ROUND, kActHSwish, MB, WGM, WGN, TM, TN>(acc, bv, lds, nhwc); break;
+  case kActHSigmoid: stage_tile<ROUND, kActHSigmoid, MB, WGM, WGN, TM, TN>(acc, bv, lds, nhwc); break;
+  case kActSigmoid: stage_tile<ROUND, kActSigmoid, MB, WGM, WGN, TM, TN>(acc, bv, lds, nhwc); break;
+  default: stage_tile<ROUND, kActNone, MB, WGM, WGN, TM, TN>(acc, bv, lds, nhwc); break;
   }
   __syncthreads();
 
@@ -311,13 +315,13 @@ __device__ __forceinline__ void tile_epilogue_bv(typename Mf<MB>::acc_t (&acc)[T
 }
 
 // Fused epilogue with the bias loaded here (the common case).
-template <int MB, int WGM, int WGN, int TM, int TN, class PixFn>
+template <bool ROUND, int MB, int WGM, int WGN, int TM, int TN, class PixFn>
 __device__ __forceinline__ void tile_epilogue(typename Mf<MB>::acc_t (&acc)[TN][TM], const ConvParams & p,
                                               _Float16 * lds, int n0, int kz, PixFn pix)
 {
   float bv[TN][Mf<MB>::NV];
   load_bias<MB, WGM, WGN, TM, TN>(p, n0, bv);
-  tile_epilogue_bv<MB, WGM, WGN, TM, TN>(acc, bv, p, lds, n0, kz, pix);
+  tile_epilogue_bv<ROUND, MB, WGM, WGN, TM, TN>(acc, bv, p, lds, n0, kz, pix);
 }
 
 }  // namespace ivh

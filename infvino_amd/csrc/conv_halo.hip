@@ -225,7 +225,7 @@ __global__ void __launch_bounds__(256) conv3x3s1_kernel(const ConvParams p)
     if (s + 1 < nsteps) step(s + 1, W1, W0);
   }
 
-  tile_epilogue<MB, WGM, WGN, TM, TN>(acc, p, lds, n0, 0, [&](int pl, int & b, int & hw) {
+  tile_epilogue<false, MB, WGM, WGN, TM, TN>(acc, p, lds, n0, 0, [&](int pl, int & b, int & hw) {
     if (pl >= TH * TW) return false;
     const int ty = idiv_small(pl, TW, inv_tw), tx = pl - ty * TW;
     const int gy = oy0 + ty, ox = ox0 + tx;

@@ -278,7 +278,7 @@ __global__ void __launch_bounds__(256, OCC) conv_igemm_kernel(const ConvParams p
       if (s + u < nk) step(s + u, u % PF, (u & 1) ? S1 : S0, (u & 1) ? S0 : S1);
   }
 
-  tile_epilogue<32, WGM, WGN, TM, TN>(acc, p, lds, n0, bz, [&](int pl, int & b, int & hw) {
+  tile_epilogue<true, 32, WGM, WGN, TM, TN>(acc, p, lds, n0, bz, [&](int pl, int & b, int & hw) {
     const unsigned pm = m0 + pl;
     if (pm >= M) return false;
     b = (int)fastdiv(pm, p.dv_hwo);

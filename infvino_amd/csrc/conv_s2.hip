@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(256) conv3x3s2_kernel(const ConvParams p)
     }
   __syncthreads();  // every wave is done with the patch: the epilogue reuses its LDS
 
-  tile_epilogue<32, WGM, WGN, 1, TN>(acc, p, lds, 0, 0, [&](int q, int & b, int & hw) {
+  tile_epilogue<false, 32, WGM, WGN, 1, TN>(acc, p, lds, 0, 0, [&](int q, int & b, int & hw) {
     if (q >= TH * TW) return false;
     const int qy = q / TW, qx = q - qy * TW;
     const int oy = oy0 + qy, ox = ox0 + qx;
