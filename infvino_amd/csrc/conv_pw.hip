@@ -161,12 +161,13 @@ __global__ void __launch_bounds__(256, 2) conv1x1_pw_kernel(const ConvParams p, 
         if (ch + 8 <= p.Cout || (ch < p.Cout && p.ypad >= ch + 8 - p.Cout)) {
           __builtin_amdgcn_raw_buffer_store_b128(q, yr, yo == kBufOOB ? kBufOOB : yo + (unsigned)ch * 2u, 0, 0);
         } else if (ch < p.Cout && yo != kBufOOB) {  // ragged last piece: the channels below Cout
-          const h8 hv = __builtin_bit_cast(h8, q);
+          // (the pieces as a vector of 16-bit integers: a bit cast of one element of a vector
+          // variable takes the vector's first bytes)
+          const u16x8 hv = __builtin_bit_cast(u16x8, q);
 #pragma unroll
           for (int e = 0; e < 8; ++e)
             if (ch + e < p.Cout)
-              __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, hv[e]), yr,
-                                                    yo + (unsigned)(ch + e) * 2u, 0, 0);
+              __builtin_amdgcn_raw_buffer_store_b16(hv[e], yr, yo + (unsigned)(ch + e) * 2u, 0, 0);
         }
       }
 #pragma unroll

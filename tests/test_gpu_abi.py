@@ -313,6 +313,30 @@ def test_abi_pointwise_planes(cin, cout, h, w, res, off):
         assert _ok(got[b], ref, f"planes {cin}->{cout} image {b}")
 
 
+@pytest.mark.parametrize("cin,cout,h,w,B,act", [
+    (8, 3, 64, 64, 15, ops.ACT_NONE), (16, 13, 59, 59, 15, ops.ACT_SILU), (51, 19, 90, 90, 14, ops.ACT_HSWISH),
+    (13, 41, 71, 71, 12, ops.ACT_RELU), (126, 63, 92, 93, 32, ops.ACT_SILU), (90, 101, 46, 47, 28, ops.ACT_SILU),
+])
+def test_abi_pointwise_ragged_outputs(cin, cout, h, w, B, act):
+    """Channels-last 1x1 convs of many pixels (the streaming kernel) whose output channels leave a
+    partial last piece: its values one by one, and the pixel's padding untouched."""
+    rng = np.random.default_rng(cin + cout)
+    d = ops.conv_desc(cin, cout, h, w, act=act)
+    x = O.f2h((rng.random(B * cin * h * w) * 2 - 1).astype(np.float32))
+    wt = O.f2h((rng.standard_normal(cout * cin) * np.sqrt(2.0 / cin)).astype(np.float32))
+    bias = O.f2h((rng.standard_normal(cout) * 0.5).astype(np.float32))
+    packed, c8 = _pack(d, wt, bias), (cout + 7) // 8 * 8
+    xd, yd = _dev(_nhwc(x, B, cin, h, w)), _dev(np.full(B * h * w * c8 + 16, 0x1234, np.uint16))
+    ops.conv2d(d, xd.data_ptr(), packed.data_ptr(), None, yd.data_ptr(), B)
+    y = _host(yd)
+    assert np.all(y[-16:] == 0x1234) and np.all(y[:-16].reshape(-1, c8)[:, cout:] == 0x1234)
+    got = _from_nhwc(y[:-16], B, cout, h, w)
+    for b in (0, B - 1):
+        ref = O.conv2d(x[b * cin * h * w:(b + 1) * cin * h * w], wt, bias, None, cin, h, w, cout, 1, 1, 0, 1, h, w, act,
+                       O.F32, 2)
+        assert _ok(got[b], ref, f"streaming 1x1 {cin}->{cout} image {b}")
+
+
 @pytest.mark.parametrize("cin,cout,h,w,k,s,B,res", [
     (256, 256, 20, 20, 3, 1, 1, False),   # 32 x 32 tiles, eight waves of nine chunks
     (128, 100, 13, 11, 3, 2, 2, True),    # the same with uneven K shares, ragged channels, residual
